@@ -31,10 +31,9 @@
 //    partials).  With arrival counters the last workgroup of a (row, kv
 //    head) to finish merges the split partials in the same launch.
 //
-//  * Generic (any dtype, head_dim <= 256, group <= 64, any page size).  A
-//    straightforward LDS-tiled implementation kept for fp32 and unusual
-//    shapes; it is the accuracy reference path on the GPU (fp32 math
-//    throughout).
+//  * Generic (any dtype, head_dim <= 256, group <= 64, any page size).  fp32
+//    products throughout (v_mfma_f32_16x16x4), K and V loaded straight into
+//    the matrix operands; also the accuracy reference path on the GPU.
 //
 // Softmax runs in base 2: scores are multiplied by scale*log2(e) and
 // exponentiated with exp2, which is the native v_exp_f32.  Partial maxima are
@@ -1276,127 +1275,371 @@ paged_decode_mfma_kernel(AttnParams p) {
 }
 
 // ===========================================================================
-// Generic kernel (fp32 math, LDS tiles)
+// Generic kernel (fp32 products on v_mfma_f32_16x16x4, any layout)
 // ===========================================================================
-constexpr int kGenericThreads = 256;
-constexpr int kGenericTile = 16;
-constexpr int kGenericMaxAcc = 32;  // group * head_dim <= 256 * 32
+// Everything the MFMA kernel above does not take: fp32 storage, other
+// head_dims, groups above 16, pages that are not a multiple of 16 tokens.
+// The call is a stream over K and V (4 flop/byte at fp32, group 8), so the
+// kernel is built to keep loads in flight: a wavefront takes 16-token tiles
+// round-robin, loads the next tile's K and V rows straight into the matrix
+// operands' registers while it computes the current one, and needs LDS only
+// for the page window and the four wavefronts' combine at the end.
+//
+// v_mfma_f32_16x16x4_f32 multiplies and accumulates in fp32.  Its operands
+// hold one float per lane (row lane & 15, k lane >> 4), and which element of
+// a row a k-step stands for is free as long as both operands agree, so both
+// tiles are loaded as whole vectors:
+//   scores  S^T[token][head]: lane (l16, q4) holds K[token l16][16 j + 4 q4
+//           + e], e = 0..3, one float4 per j; k-step (j, e) pairs it with
+//           Q[head l16] at the same element.  Result register r: token
+//           4 q4 + r of head l16 -- which is the B operand of P.V as it is.
+//   P.V     O^T[dim][head]: k-step r takes tokens 4 q4 + r, so lane (l16,
+//           q4) holds V[token 4 q4 + r][kVec l16 .. + kVec) of every 16 kVec
+//           dims: 16 lanes read a head's row of V whole.  Element n of that
+//           vector is row l16 of output block n.
+// Heads are padded to 16 columns with copies of the last one; groups above
+// 16 walk the tokens once per 16 heads.
+//
+// Bound by the loads in flight and, below that, by the two chains of matrix
+// products per tile (2 x 512 cycles at D 64; fp32 runs at 1/16 of the bf16
+// rate).  Four wavefronts per workgroup: eight made the fixed cost of a
+// short partition 8 us against 4.6.  The loop head waits for one of the two
+// register sets only because every iteration loads both (27.5 us; 34 us with
+// the next tile's loads under a branch).  MI355X, fp32, 32/4 heads, D 64, 32
+// ragged rows to 2048 tokens: 512 -> 26.6 us per call (2.7 TB/s; the form
+// this replaces staged 16-token tiles in LDS and ran them on the VALU); 8
+// rows of 1000 10.1 us; 16 rows to 2048 at 32/8 heads, D 128 54 us.
+constexpr int kGenericMaxItems = 8192; // group * head_dim
+constexpr int kGenericWindow = 1024;   // tokens per page window
+constexpr int kGenericWaves = 4;       // wavefronts per workgroup
+// Partial results the wavefronts leave in LDS for the final sum (at most
+// 33 KB, beside the 33 KB of a group above 16).
+template <int DT>
+constexpr int generic_slices() { return DT <= 64 ? 4 : (DT <= 192 ? 2 : 1); }
 
-template <typename T>
-__global__ void __launch_bounds__(kGenericThreads)
+// How a kernel instance reads four consecutive elements: whole rows of
+// exactly DT elements (kRowsExact), vectors that may lie past head_dim
+// (kRowsPadded, head_dim % 4 == 0), or single elements (kRowsScalar: any
+// head_dim, any alignment).
+enum GenericRows : int { kRowsExact = 0, kRowsPadded = 1, kRowsScalar = 2 };
+
+template <typename T, int N>
+struct alignas(sizeof(T) * N) GenericVec {
+  T v[N];
+};
+
+template <typename T, int DT, int ROWS>
+__global__ void __launch_bounds__(64 * kGenericWaves, DT <= 64 ? 3 : 1)
 paged_decode_generic_kernel(AttnParams p) {
+  constexpr int kWaves = kGenericWaves;
+  constexpr int kSlices = generic_slices<DT>();
+  constexpr int KJ = DT / 16;              // float4 pieces of a K row per lane
+  constexpr int kVec = DT == 32 ? 2 : 4;   // consecutive dims per lane of a V row
+  constexpr int VB = DT / (16 * kVec);     // such vectors per V row
+  constexpr int NB = VB * kVec;            // 16-dim output blocks
+  constexpr int kSets = DT <= 128 ? 2 : 1; // tiles in flight (registers)
+  using VK = GenericVec<T, 4>;
+  using VV = GenericVec<T, kVec>;
   extern __shared__ __attribute__((aligned(16))) unsigned char generic_smem[];
-  float *smem = reinterpret_cast<float *>(generic_smem);
   const int D = p.head_dim;
   const int G = p.group;
-  float *ks = smem;                            // [tile][D + 1]
-  float *vs = ks + kGenericTile * (D + 1);     // [tile][D]
-  float *sc = vs + kGenericTile * D;           // [G][tile]
-  float *m_run = sc + G * kGenericTile;        // [G]
-  float *l_run = m_run + G;                    // [G]
-  float *alpha = l_run + G;                    // [G]
-  int *tok_ok = reinterpret_cast<int *>(alpha + G);  // [tile]
+  const int pitch = D + 1;
+  float *slices = reinterpret_cast<float *>(generic_smem);  // [kSlices][16][D + 1] numerators
+  float *wave_max = slices + kSlices * 16 * pitch;          // [waves][16]
+  float *wave_sums = wave_max + kWaves * 16;                // [waves][16]
+  float *head_max = wave_sums + kWaves * 16;                // [G]
+  float *head_sum = head_max + G;                           // [G]
+  float *result = head_sum + G;                             // [G][D + 1], groups above 16 only
+  int32_t *window = reinterpret_cast<int32_t *>(result + (G > 16 ? G * pitch : 0));
 
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15;
+  const int q4 = lane >> 4;
   const int32_t b = blockIdx.x / p.kv_heads;
   const int32_t kvh = blockIdx.x - b * p.kv_heads;
   const int32_t split = blockIdx.y;
-  const int32_t ctx = clamp_context(p, b);
   const int32_t s0 = split * p.split_size;
+  const int32_t *table = p.block_tables + static_cast<int64_t>(b) * p.table_width;
+  auto logical_of = [&](int32_t t) { return p.page_shift >= 0 ? t >> p.page_shift : t / p.block_size; };
+  // The first page window does not wait for the row's length: its entries
+  // are bounded by the split and the table.
+  {
+    const int32_t first = logical_of(s0);
+    const int32_t last = min(logical_of(s0 + min(p.split_size, kGenericWindow) - 1), p.table_width - 1);
+    for (int32_t i = threadIdx.x; i <= last - first; i += 64 * kWaves) window[i] = table[first + i];
+  }
+  const int32_t ctx = clamp_context(p, b);
   if (s0 >= ctx) {
-    if (split == 0) zero_rows<T>(p, b, kvh * p.group, p.group);
+    if (split == 0) zero_rows<T>(p, b, kvh * G, G);
     return;
   }
   const int32_t s1 = min(s0 + p.split_size, ctx);
-  const int32_t *table = p.block_tables + static_cast<int64_t>(b) * p.table_width;
   const T *q = static_cast<const T *>(p.query) +
                (static_cast<int64_t>(b) * p.query_heads + static_cast<int64_t>(kvh) * G) * D;
   const T *kbase = static_cast<const T *>(p.key_cache) + static_cast<int64_t>(kvh) * D;
   const T *vbase = static_cast<const T *>(p.value_cache) + static_cast<int64_t>(kvh) * D;
+  const int64_t row_elems = static_cast<int64_t>(p.kv_heads) * D;
 
-  for (int g = threadIdx.x; g < G; g += blockDim.x) {
-    m_run[g] = kNegInf;
-    l_run[g] = 0.f;
-  }
-  float acc[kGenericMaxAcc];
+  // N elements [d, d + N) of a row that starts at `row`; zeros past head_dim.
+  auto load_row = [&](const T *row, int d, auto tag) {
+    using V = decltype(tag);
+    constexpr int N = sizeof(V) / sizeof(T);
+    V out;
+    if constexpr (ROWS == kRowsExact) {
+      if constexpr (sizeof(V) == 16) {
+        out = load_stream16<V>(row + d);
+      } else {
+        out = *reinterpret_cast<const V *>(row + d);
+      }
+    } else if constexpr (ROWS == kRowsPadded) {
+      if (d < D) {
+        out = *reinterpret_cast<const V *>(row + d);
+      } else {
 #pragma unroll
-  for (int i = 0; i < kGenericMaxAcc; ++i) acc[i] = 0.f;
+        for (int e = 0; e < N; ++e) out.v[e] = T(0);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; ++e) out.v[e] = d + e < D ? row[d + e] : T(0);
+    }
+    return out;
+  };
 
-  for (int32_t t0 = s0; t0 < s1; t0 += kGenericTile) {
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < kGenericTile * D; idx += blockDim.x) {
-      const int tt = idx / D;
-      const int d = idx - tt * D;
-      const int32_t t = t0 + tt;
-      int64_t off = -1;
-      if (t < s1) off = token_offset(p, table, t);
-      float kv = 0.f, vv = 0.f;
-      if (off >= 0) {
-        kv = to_float(kbase[off + d]);
-        vv = to_float(vbase[off + d]);
+  for (int32_t h0 = 0; h0 < G; h0 += 16) {  // uniform: one pass for groups up to 16
+    float qf[KJ][4];  // Q[head h0 + l16][16 j + 4 q4 + e]
+    {
+      const T *qrow = q + static_cast<int64_t>(min(h0 + l16, G - 1)) * D;
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) {
+        const VK v = load_row(qrow, 16 * j + 4 * q4, VK{});
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qf[j][e] = to_float(v.v[e]);
       }
-      ks[tt * (D + 1) + d] = kv;
-      vs[tt * D + d] = vv;
-      if (d == 0) tok_ok[tt] = off >= 0;
     }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < G * kGenericTile; idx += blockDim.x) {
-      const int g = idx / kGenericTile;
-      const int tt = idx - g * kGenericTile;
-      float s = kNegInf;
-      if (tok_ok[tt]) {
-        float dot = 0.f;
-        for (int d = 0; d < D; ++d) dot += to_float(q[g * D + d]) * ks[tt * (D + 1) + d];
-        s = dot * p.scale_log2;
+    f32x4 acc[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = kNegInf;  // reference max of head l16 (base 2, scaled)
+    float l_run = 0.f;      // lane-partial sum of head l16
+
+    VK kr[kSets][KJ];
+    VV vr[kSets][4][VB];
+    uint32_t present[kSets];  // bit t: token t of the tile has a page
+
+    // Loads of the 16-token tile at t0 (tokens [t0, min(t0 + 16, t1))).
+    // Absent tokens read the query row, whose bytes are masked below.
+    auto load_tile = [&](int32_t t0, int32_t t1, int32_t first_page, int set) {
+      const int32_t t = t0 + l16;
+      int64_t row = -1;
+      if (t < t1) {
+        const int32_t logical = logical_of(t);
+        const int32_t page = window[logical - first_page];
+        if (page >= 0 && page < p.num_blocks)
+          row = static_cast<int64_t>(page) * p.block_size + (t - logical * p.block_size);
       }
-      sc[idx] = s;
-    }
-    __syncthreads();
-    for (int g = threadIdx.x; g < G; g += blockDim.x) {
-      float mx = kNegInf;
-      for (int tt = 0; tt < kGenericTile; ++tt) mx = fmaxf(mx, sc[g * kGenericTile + tt]);
-      const float m_new = fmaxf(m_run[g], mx);
-      float a = 1.f, sum = 0.f;
-      if (m_new != kNegInf) {
-        a = exp2f(m_run[g] - m_new);
-        for (int tt = 0; tt < kGenericTile; ++tt) {
-          const float pr = exp2f(sc[g * kGenericTile + tt] - m_new);
-          sc[g * kGenericTile + tt] = pr;
-          sum += pr;
+      present[set] = static_cast<uint32_t>(__ballot(row >= 0)) & 0xffffu;
+      const T *krow = row >= 0 ? kbase + row * row_elems : q;
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) kr[set][j] = load_row(krow, 16 * j + 4 * q4, VK{});
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int src = 4 * q4 + r;  // the lane that holds token 4 q4 + r
+        const uint32_t lo = static_cast<uint32_t>(__shfl(static_cast<int>(row & 0xffffffff), src, 64));
+        const int32_t hi = __shfl(static_cast<int>(row >> 32), src, 64);
+        const int64_t vrow_at = static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | lo);
+        const T *vrow = vrow_at >= 0 ? vbase + vrow_at * row_elems : q;
+#pragma unroll
+        for (int vb = 0; vb < VB; ++vb)
+          vr[set][r][vb] = load_row(vrow, 16 * kVec * vb + kVec * l16, VV{});
+      }
+    };
+    auto compute_tile = [&](int set) {
+      // Two accumulators halve the chain of dependent products.
+      f32x4 se = f32x4{0.f, 0.f, 0.f, 0.f}, so = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          se = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(kr[set][j].v[e]), qf[j][e], se, 0, 0, 0);
+          so = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(kr[set][j].v[e + 1]), qf[j][e + 1], so, 0, 0, 0);
+        }
+      }
+      float sc[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool ok = (present[set] >> (4 * q4 + r)) & 1u;
+        sc[r] = ok ? (se[r] + so[r]) * p.scale_log2 : kNegInf;
+      }
+      float mx = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+      if (__ballot(mx > m_run + kRescaleThreshold) != 0) {  // uniform
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = m_new == kNegInf ? 1.f : fast_exp2(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[n] *= alpha;
+      }
+      const float m_ref = m_run == kNegInf ? 0.f : m_run;
+      float pr[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pr[r] = fast_exp2(sc[r] - m_ref);
+        l_run += pr[r];
+      }
+      const bool whole = present[set] == 0xffffu;  // uniform
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool ok = whole || ((present[set] >> (4 * q4 + r)) & 1u);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          // Absent tokens' stand-in values are cleared: 0 * inf is not 0.
+          const float v = ok ? to_float(vr[set][r][n / kVec].v[n % kVec]) : 0.f;
+          acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, pr[r], acc[n], 0, 0, 0);
+        }
+      }
+    };
+
+    for (int32_t seg = s0; seg < s1; seg += kGenericWindow) {
+      const int32_t seg_end = min(seg + kGenericWindow, s1);
+      const int32_t first_page = logical_of(seg);
+      const int32_t pages = logical_of(seg_end - 1) - first_page + 1;
+      __syncthreads();  // the previous window's (or pass's) reads are done
+      if (seg != s0 || h0 != 0) {
+        for (int32_t i = threadIdx.x; i < pages; i += 64 * kWaves) window[i] = table[first_page + i];
+        __syncthreads();
+      }
+      const int32_t step = 16 * kWaves;
+      const int32_t first = seg + 16 * wave;
+      if (first >= seg_end) continue;  // wavefront-uniform; no barrier inside the walk
+      const int32_t last = first + (seg_end - 1 - first) / step * step;
+      if constexpr (kSets == 2) {
+        // Every iteration issues both sets' loads (past the last tile that
+        // tile again, unused): loads issued on some paths only would make
+        // each wait drain both sets.
+        load_tile(first, seg_end, first_page, 0);
+        for (int32_t t0 = first; t0 <= last; t0 += 2 * step) {
+          load_tile(min(t0 + step, last), seg_end, first_page, 1);
+          compute_tile(0);
+          load_tile(min(t0 + 2 * step, last), seg_end, first_page, 0);
+          if (t0 + step <= last) compute_tile(1);  // uniform
         }
       } else {
-        for (int tt = 0; tt < kGenericTile; ++tt) sc[g * kGenericTile + tt] = 0.f;
+        for (int32_t t0 = first; t0 <= last; t0 += step) {
+          load_tile(t0, seg_end, first_page, 0);
+          compute_tile(0);
+        }
       }
-      l_run[g] = l_run[g] * a + sum;
-      m_run[g] = m_new;
-      alpha[g] = a;
+    }
+
+    // The wavefronts' states meet in LDS: common maximum, then the scaled
+    // numerators added in wavefront order.
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    if (q4 == 0) {
+      wave_max[wave * 16 + l16] = m_run;
+      wave_sums[wave * 16 + l16] = l_run;
     }
     __syncthreads();
+    float m_all = kNegInf;
 #pragma unroll
-    for (int i = 0; i < kGenericMaxAcc; ++i) {
-      const int idx = threadIdx.x + i * kGenericThreads;
-      if (idx < G * D) {
-        const int g = idx / D;
-        const int d = idx - g * D;
-        float a = acc[i] * alpha[g];
-        for (int tt = 0; tt < kGenericTile; ++tt) a += sc[g * kGenericTile + tt] * vs[tt * D + d];
-        acc[i] = a;
+    for (int w = 0; w < kWaves; ++w) m_all = fmaxf(m_all, wave_max[w * 16 + l16]);
+    auto factor = [&](float m) { return m == kNegInf ? 0.f : fast_exp2(m - m_all); };
+    float l_all = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) l_all += wave_sums[w * 16 + l16] * factor(wave_max[w * 16 + l16]);
+    const float own = factor(m_run);
+    const bool head_ok = h0 + l16 < G;
+    if (wave == 0 && q4 == 0 && head_ok) {
+      head_max[h0 + l16] = m_all;
+      head_sum[h0 + l16] = l_all;
+    }
+    // Wavefront w adds to slice w % kSlices, kSlices wavefronts at a time.
+    float *hrow = slices + ((wave % kSlices) * 16 + l16) * pitch;
+#pragma unroll
+    for (int w0 = 0; w0 < kWaves; w0 += kSlices) {
+      if (wave / kSlices == w0 / kSlices && head_ok) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int d = 16 * kVec * (n / kVec) + kVec * (4 * q4 + r) + n % kVec;
+            if (ROWS == kRowsExact || d < D)
+              hrow[d] = w0 == 0 ? acc[n][r] * own : __builtin_fmaf(acc[n][r], own, hrow[d]);
+          }
       }
+      __syncthreads();
+    }
+    if (G > 16) {  // the next pass reuses the slices
+      for (int i = threadIdx.x; i < 16 * D; i += 64 * kWaves) {
+        const int g = i / D;
+        const int d = i - g * D;
+        if (h0 + g >= G) break;
+        float sum = 0.f;
+#pragma unroll
+        for (int sl = 0; sl < kSlices; ++sl) sum += slices[(sl * 16 + g) * pitch + d];
+        result[(h0 + g) * pitch + d] = sum;
+      }
+      __syncthreads();
     }
   }
-  __syncthreads();
-  finish<T, kGenericMaxAcc>(p, b, kvh * G, G, static_cast<int64_t>(b) * p.kv_heads + kvh, split, ctx,
-                            [&](int k, int idx, float &m, float &l, float &num) {
-                              const int g = idx / D;
-                              m = m_run[g];
-                              l = l_run[g];
-                              num = acc[k];
-                            });
+  finish<T, kGenericMaxItems / (64 * kWaves)>(
+      p, b, kvh * G, G, static_cast<int64_t>(b) * p.kv_heads + kvh, split, ctx,
+      [&](int, int idx, float &m, float &l, float &num) {
+        const int g = idx / D;
+        const int d = idx - g * D;
+        m = head_max[g];
+        l = head_sum[g];
+        if (G > 16) {
+          num = result[g * pitch + d];
+        } else {
+          num = 0.f;
+#pragma unroll
+          for (int sl = 0; sl < kSlices; ++sl) num += slices[(sl * 16 + g) * pitch + d];
+        }
+      });
 }
 
-size_t generic_lds_bytes(int D, int G) {
-  return sizeof(float) * (static_cast<size_t>(kGenericTile) * (D + 1) +
-                          static_cast<size_t>(kGenericTile) * D + static_cast<size_t>(G) * kGenericTile +
-                          3 * static_cast<size_t>(G) + kGenericTile);
+// Page window entries: every page of kGenericWindow tokens, one page more
+// when the window starts inside a page.
+size_t generic_lds_bytes(int D, int G, int block_size, int slices) {
+  const size_t pages = static_cast<size_t>(kGenericWindow / block_size) + 2;
+  const size_t pitch = static_cast<size_t>(D) + 1;
+  return sizeof(float) * (static_cast<size_t>(slices) * 16 * pitch + 2 * static_cast<size_t>(kGenericWaves) * 16 +
+                          2 * static_cast<size_t>(G) + (G > 16 ? static_cast<size_t>(G) * pitch : 0) + pages);
+}
+
+// Whole vectors where every K, V and Q row starts on a vector of four
+// elements, single elements otherwise.
+template <typename T, int DT, int ROWS>
+void launch_generic_form(const AttnParams &p, dim3 grid, hipStream_t stream) {
+  hipLaunchKernelGGL((paged_decode_generic_kernel<T, DT, ROWS>), grid, dim3(64 * kGenericWaves),
+                     generic_lds_bytes(p.head_dim, p.group, p.block_size, generic_slices<DT>()), stream, p);
+}
+
+template <typename T>
+void launch_generic(const AttnParams &p, dim3 grid, hipStream_t stream) {
+  const int D = p.head_dim;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p.query) | reinterpret_cast<uintptr_t>(p.key_cache) |
+                       reinterpret_cast<uintptr_t>(p.value_cache);
+  const bool vectors = D % 4 == 0 && at % (4 * sizeof(T)) == 0;
+  if constexpr (sizeof(T) == 4) {
+    if (vectors && D == 32) return launch_generic_form<T, 32, kRowsExact>(p, grid, stream);
+    if (vectors && D == 64) return launch_generic_form<T, 64, kRowsExact>(p, grid, stream);
+    if (vectors && D == 128) return launch_generic_form<T, 128, kRowsExact>(p, grid, stream);
+    if (vectors && D == 256) return launch_generic_form<T, 256, kRowsExact>(p, grid, stream);
+  }
+  if (vectors) {
+    if (D <= 64) return launch_generic_form<T, 64, kRowsPadded>(p, grid, stream);
+    if (D <= 128) return launch_generic_form<T, 128, kRowsPadded>(p, grid, stream);
+    if (D <= 192) return launch_generic_form<T, 192, kRowsPadded>(p, grid, stream);
+    return launch_generic_form<T, 256, kRowsPadded>(p, grid, stream);
+  }
+  if (D <= 64) return launch_generic_form<T, 64, kRowsScalar>(p, grid, stream);
+  if (D <= 128) return launch_generic_form<T, 128, kRowsScalar>(p, grid, stream);
+  return launch_generic_form<T, 256, kRowsScalar>(p, grid, stream);
 }
 
 // ===========================================================================
@@ -1739,23 +1982,13 @@ int32_t launch_split_stage(const AttnParams &p, int32_t dtype, int32_t flags, hi
       launch_mfma_dim<_Float16>(q, mgrid, stream);
     return check_launch("paged_gqa_decode (mfma)");
   }
-  if (p.group > 64 || p.group * p.head_dim > kGenericThreads * kGenericMaxAcc)
+  if (p.group > 64 || p.group * p.head_dim > kGenericMaxItems)
     return fail(TF_ERROR_UNSUPPORTED,
                 "generic attention supports group <= 64 and group * head_dim <= 8192");
-  const size_t lds = generic_lds_bytes(p.head_dim, p.group);
   switch (dtype) {
-    case TF_DTYPE_FLOAT32:
-      hipLaunchKernelGGL(paged_decode_generic_kernel<float>, grid, dim3(kGenericThreads), lds,
-                         stream, p);
-      break;
-    case TF_DTYPE_FLOAT16:
-      hipLaunchKernelGGL(paged_decode_generic_kernel<_Float16>, grid, dim3(kGenericThreads), lds,
-                         stream, p);
-      break;
-    default:
-      hipLaunchKernelGGL(paged_decode_generic_kernel<__bf16>, grid, dim3(kGenericThreads), lds,
-                         stream, p);
-      break;
+    case TF_DTYPE_FLOAT32: launch_generic<float>(p, grid, stream); break;
+    case TF_DTYPE_FLOAT16: launch_generic<_Float16>(p, grid, stream); break;
+    default: launch_generic<__bf16>(p, grid, stream); break;
   }
   return check_launch("paged_gqa_decode (generic)");
 }
