@@ -557,6 +557,105 @@ int32_t tf_prefill_attention(const void *q, int64_t q_row_stride, const void *k,
                              void *stream);
 
 /*
+ * y = round(x @ weight^T) for prefill's packed prompt rows (any m), or with
+ * `partials` the fp32 slice sums partials[s][i][j] of `splits` contiguous
+ * slices of K (of its C 64-wide chunks, [s C / splits, (s + 1) C / splits)), or
+ * with `swiglu` the activation of a stacked gate|up weight of 2 n rows:
+ *   y[i][j] = round(swiglu(round(x[i] . w[j]), round(x[i] . w[n + j]))).
+ * K % 64 == 0, n % 4 == 0, 16-byte aligned x, weight and partials rows and
+ * 8-byte aligned y rows, fp16/bf16; every slice must fill the load ring of
+ * its tile (2 to 4 chunks).  `tile` (0: chosen from the sizes, else 1 to 10)
+ * names the workgroup tile.  Replaces the torch GEMMs of prefill's nn.Linear
+ * projections (tensorforge/model/layers.py:88-95, 144-158;
+ * runtime/prefill.py:90-135).
+ */
+int32_t tf_prefill_linear(const void *x, int64_t x_row_stride, const void *weight,
+                          int64_t weight_row_stride, void *y, int64_t y_row_stride,
+                          float *partials, int32_t m, int32_t n, int32_t k, int32_t splits,
+                          int32_t swiglu, int32_t tile, int32_t dtype, void *stream);
+
+/*
+ * K slices that tf_prefill_linear runs fastest with for these sizes when its
+ * consumer can add slice sums (1 to 4; 1: write the rounded product), or 0
+ * where K does not suit it.
+ */
+int32_t tf_prefill_linear_splits(int32_t m, int32_t n, int32_t k);
+
+/*
+ * tf_rope_kv_append over the slice sums of a K-split q|k|v projection,
+ * partials [splits][batch][(query_heads + 2 kv_heads) * head_dim]: the sums
+ * are added in slice order and rounded once, then rotated and written as
+ * there; key_out and value_out are the dense rotated keys and values.
+ * head_dim % 16 == 0, 16-byte aligned buffers, fp16/bf16.
+ */
+int32_t tf_rope_kv_append_partials(
+    const float *partials, int32_t splits, const int64_t *positions, const void *cos_table,
+    const void *sin_table, int32_t table_rows, void *query_out, void *key_out, void *value_out,
+    void *key_cache, void *value_cache, const int32_t *physical_blocks,
+    const int32_t *block_offsets, const int32_t *active_mask, int32_t batch, int32_t query_heads,
+    int32_t kv_heads, int32_t head_dim, int32_t num_blocks, int32_t block_size, int32_t dtype,
+    void *stream);
+
+/*
+ * One decoder layer of a packed prefill, its launches enqueued in one call:
+ * the q|k|v projection of h, RoPE with the page writes, the prompts' causal
+ * attention, the o projection added to the residual with the post-attention
+ * RMSNorm, gate|up with SwiGLU, and the down projection added to the residual
+ * with the next RMSNorm.  Projections run as tf_prefill_linear (K slices
+ * where that is faster, summed by their consumers); the results are those of
+ * the entry points called one by one.
+ *   h [tokens][hidden] and residual [tokens][hidden] are the layer's inputs
+ *   (normalised and not) and are overwritten with its outputs; act [tokens]
+ *   [intermediate], query and context [tokens][query_heads * head_dim], key
+ *   and value [tokens][kv_heads * head_dim], rows [tokens][max(hidden,
+ *   (query_heads + 2 kv_heads) * head_dim)] and second_residual [tokens]
+ *   [hidden] are scratch, all dense; partials holds partial_floats fp32.
+ * Replaces the layer loop of tensorforge/runtime/prefill.py:90-135.
+ */
+typedef struct tf_prefill_layer_args {
+  void *h;
+  void *residual;
+  void *second_residual;
+  void *rows;
+  void *query;
+  void *key;
+  void *value;
+  void *context;
+  void *act;
+  float *partials;
+  int64_t partial_floats;
+  const void *qkv_weight;
+  const void *o_weight;
+  const void *gate_up_weight;
+  const void *down_weight;
+  const void *post_norm;
+  const void *next_norm;
+  const void *cos_table;
+  const void *sin_table;
+  void *key_cache;
+  void *value_cache;
+  const int64_t *positions;
+  const int32_t *physical_blocks;
+  const int32_t *block_offsets;
+  const int32_t *active_mask;
+  const int32_t *tiles;
+  int32_t table_rows;
+  int32_t num_tiles;
+  int32_t tokens;
+  int32_t hidden;
+  int32_t intermediate;
+  int32_t query_heads;
+  int32_t kv_heads;
+  int32_t head_dim;
+  int32_t num_blocks;
+  int32_t block_size;
+  float eps;
+  float scale;
+  int32_t dtype;
+} tf_prefill_layer_args;
+int32_t tf_prefill_layer(const tf_prefill_layer_args *args, void *stream);
+
+/*
  * Measurement only: stream `bytes` (a positive multiple of 16) of the
  * 16-byte aligned `buffer` from HBM with 16-byte nontemporal loads.
  * `workgroups` workgroups of `waves` (1..16) wavefronts each read one

@@ -41,6 +41,26 @@ _i32 = ctypes.c_int32
 _i64 = ctypes.c_int64
 _f32 = ctypes.c_float
 
+
+class PrefillLayerArgs(ctypes.Structure):
+    """tf_prefill_layer_args of the header, field for field."""
+
+    _fields_ = (
+        [(name, _p) for name in (
+            "h", "residual", "second_residual", "rows", "query", "key", "value", "context", "act",
+            "partials")]
+        + [("partial_floats", _i64)]
+        + [(name, _p) for name in (
+            "qkv_weight", "o_weight", "gate_up_weight", "down_weight", "post_norm", "next_norm",
+            "cos_table", "sin_table", "key_cache", "value_cache", "positions", "physical_blocks",
+            "block_offsets", "active_mask", "tiles")]
+        + [(name, _i32) for name in (
+            "table_rows", "num_tiles", "tokens", "hidden", "intermediate", "query_heads",
+            "kv_heads", "head_dim", "num_blocks", "block_size")]
+        + [("eps", _f32), ("scale", _f32), ("dtype", _i32)]
+    )
+
+
 # name -> argument types, in header order.
 SIGNATURES: dict[str, tuple[Any, ...]] = {
     "tf_last_error": (),
@@ -117,6 +137,15 @@ SIGNATURES: dict[str, tuple[Any, ...]] = {
     "tf_linear_kswiglu_norm": (_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _f32, _i32, _p),
     "tf_linear_kstream_residual": (_p, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32,
                                    _i32, _p),
+    "tf_prefill_linear": (_p, _i64, _p, _i64, _p, _i64, _p, _i32, _i32, _i32, _i32, _i32, _i32,
+                          _i32, _p),
+    "tf_prefill_linear_splits": (_i32, _i32, _i32),
+    "tf_rope_kv_append_partials": (
+        _p, _i32, _p, _p, _p, _i32,  # partials, splits, positions, cos, sin, table rows
+        _p, _p, _p, _p, _p, _p, _p, _p,  # query/key/value out, caches, pages, offsets, active
+        _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p,  # batch .. block size, dtype, stream
+    ),
+    "tf_prefill_layer": (ctypes.POINTER(PrefillLayerArgs), _p),
     "tf_prefill_attention": (_p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i32, _i32, _i32, _i32,
                              _f32, _i32, _i32, _p),
 }

@@ -44,7 +44,7 @@ DEVICE_FLAGS = (
 # AGPRs and copies to VGPRs around every VALU use (the online softmax's
 # rescale, the split-K epilogue): the VGPR form of the MFMA instructions
 # (gfx950 reads and writes C/D in VGPRs) removes those copies.
-VGPR_MFMA_SOURCES = {"tf_prefill_attention.hip", "tf_linear_splitk.hip"}
+VGPR_MFMA_SOURCES = {"tf_prefill_attention.hip", "tf_prefill_linear.hip", "tf_linear_splitk.hip"}
 VGPR_MFMA_FLAGS = ("-mllvm", "-amdgpu-mfma-vgpr-form")
 
 

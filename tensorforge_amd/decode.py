@@ -75,6 +75,8 @@ from tensorforge_amd.kernels.linear import (
     default_splits,
     fold_norm_gain,
     linear_partials_supported,
+    prefill_linear,
+    prefill_linear_supported,
 )
 from tensorforge_amd.kernels.ops import residual_rms_norm_partials
 from tensorforge_amd.kernels.prefill import (
@@ -605,6 +607,130 @@ def _validate_prompt(weights: DecoderWeights, cache: PagedKVCache, request_id: s
         raise ValueError("prompt exceeds the model's RoPE table")
 
 
+# Prefills of at most this many tokens run their projections on the library's
+# own prefill GEMM, one native call per layer; longer ones keep hipBLASLt for
+# all but the gate|up projection (MI355X, TinyLlama: at 2000 rows qkv / o /
+# down 27.6 / 22.1 / 54.6 us against 27.2 / 20.9 / 46.3, at 8058 rows 85 / 52 /
+# 133 against 74 / 61 / 157; gate|up with its SwiGLU 433 against 346).
+PREFILL_NATIVE_TOKENS = 2048
+
+
+def _stage_prefill(cache: PagedKVCache, prompts: dict[str, list[int]], bounds: np.ndarray,
+                   tiles: np.ndarray) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    """The controls of a packed prefill, in one host-to-device copy: int64
+    rows (token ids, positions, -1 per token: the ids come from the host),
+    the last token of each prompt, int32 rows (pages, offsets, active) and
+    the attention work list."""
+
+    total = int(bounds[-1])
+    block_size = cache.config.block_size
+    words = 3 * total + len(prompts)
+    host = torch.empty(8 * words + 4 * (3 * total + tiles.size), dtype=torch.uint8, pin_memory=True)
+    view = host.numpy()
+    longs = view[:24 * total].view(np.int64).reshape(3, total)
+    view[24 * total:8 * words].view(np.int64)[:] = bounds[1:] - 1
+    ints = view[8 * words:8 * words + 12 * total].view(np.int32).reshape(3, total)
+    view[8 * words + 12 * total:].view(np.int32)[:] = tiles.reshape(-1)
+    longs[2] = -1
+    ints[2] = 1
+    for i, (request_id, prompt) in enumerate(prompts.items()):
+        lo, hi = bounds[i], bounds[i + 1]
+        positions = np.arange(hi - lo, dtype=np.int64)
+        pages = np.asarray(cache.page_list(request_id)[0], dtype=np.int32)
+        longs[0, lo:hi] = prompt
+        longs[1, lo:hi] = positions
+        ints[0, lo:hi] = pages[positions // block_size]
+        ints[1, lo:hi] = positions % block_size
+    # The pinned block goes back to torch's host allocator with the copy's
+    # stream recorded, so it is not reused before the copy has run.
+    device = host.to(cache.config.device, non_blocking=True)
+    return (device[:24 * total].view(torch.int64).view(3, total),
+            device[24 * total:8 * words].view(torch.int64),
+            device[8 * words:8 * words + 12 * total].view(torch.int32).view(3, total),
+            device[8 * words + 12 * total:].view(torch.int32).view(-1, 3))
+
+
+class _NativePrefill:
+    """Layers of one packed prefill as single native calls
+    (tf_prefill_layer), with the scratch they share."""
+
+    def __init__(self, weights: DecoderWeights, cache: PagedKVCache, total: int,
+                 positions: Tensor, ints: Tensor, tiles: Tensor) -> None:
+        config = weights.config
+        hq, hkv, d = config.num_attention_heads, config.num_key_value_heads, config.head_dim
+        hidden, inter = config.hidden_size, config.intermediate_size
+        self.cache = cache
+        self.library = _native.library()
+        self.stream = _native.current_stream(cache.config.device)
+        qkv_width = (hq + 2 * hkv) * d
+        self.shapes = {"qkv": (qkv_width, hidden), "o_proj": (hidden, hq * d),
+                       "gate_up": (2 * inter, hidden), "down": (hidden, inter),
+                       "post_norm": (hidden,)}
+        floats = max(self.library.tf_prefill_linear_splits(total, n, k) * total * n
+                     for n, k in (self.shapes["qkv"], self.shapes["o_proj"], self.shapes["down"]))
+        widths = {"second_residual": hidden, "rows": max(hidden, qkv_width), "query": hq * d,
+                  "key": hkv * d, "value": hkv * d, "context": hq * d, "act": inter}
+        device, dtype = cache.config.device, cache.config.dtype
+        self.scratch = {name: torch.empty((total, width), dtype=dtype, device=device)
+                        for name, width in widths.items()}
+        self.scratch["partials"] = torch.empty(floats, dtype=torch.float32, device=device)
+        self.args = _native.PrefillLayerArgs(
+            **{name: tensor.data_ptr() for name, tensor in self.scratch.items()},
+            partial_floats=floats, cos_table=weights.rope_cos.data_ptr(),
+            sin_table=weights.rope_sin.data_ptr(), positions=positions.data_ptr(),
+            physical_blocks=ints[0].data_ptr(), block_offsets=ints[1].data_ptr(),
+            active_mask=ints[2].data_ptr(), tiles=tiles.data_ptr(),
+            table_rows=weights.rope_cos.shape[0], num_tiles=tiles.shape[0], tokens=total,
+            hidden=hidden, intermediate=inter, query_heads=hq, kv_heads=hkv, head_dim=d,
+            num_blocks=cache.config.num_blocks, block_size=cache.config.block_size,
+            eps=config.rms_norm_eps, scale=d ** -0.5, dtype=_native.dtype_code(dtype))
+
+    @staticmethod
+    def supported(weights: DecoderWeights, cache: PagedKVCache, total: int) -> bool:
+        """Whether a prefill of ``total`` tokens can run layers this way: the
+        geometry's projections, attention and norms all have kernels for it."""
+
+        config = weights.config
+        hq, hkv, d = config.num_attention_heads, config.num_key_value_heads, config.head_dim
+        h, f = config.hidden_size, config.intermediate_size
+        return (0 < total <= PREFILL_NATIVE_TOKENS
+                and prefill_attention_supported(cache.config.dtype, hq, hkv, d) and h <= 16384
+                and min(h, f, hq * d) >= 256 and h % 64 == f % 64 == hq * d % 64 == hkv * d % 8 == 0
+                and _dense(weights.rope_cos, (weights.rope_cos.shape[0], d), cache)
+                and _dense(weights.rope_sin, tuple(weights.rope_cos.shape), cache))
+
+    def run(self, index: int, layer: LayerWeights, next_norm: Tensor, h: Tensor,
+            residual: Tensor) -> bool:
+        """Layer ``index`` over h and residual, in place; False (and nothing
+        done) where a tensor is not one the native call takes."""
+
+        tensors = {name: getattr(layer, name) for name in self.shapes}
+        rows = (self.args.tokens, self.args.hidden)
+        if not (all(_dense(tensors[name], shape, self.cache) for name, shape in self.shapes.items())
+                and _dense(next_norm, self.shapes["post_norm"], self.cache)
+                and _dense(h, rows, self.cache) and _dense(residual, rows, self.cache)):
+            return False
+        args = self.args
+        args.h = h.data_ptr()
+        args.residual = residual.data_ptr()
+        args.qkv_weight = tensors["qkv"].data_ptr()
+        args.o_weight = tensors["o_proj"].data_ptr()
+        args.gate_up_weight = tensors["gate_up"].data_ptr()
+        args.down_weight = tensors["down"].data_ptr()
+        args.post_norm = tensors["post_norm"].data_ptr()
+        args.next_norm = next_norm.data_ptr()
+        args.key_cache = self.cache.key_cache[index].data_ptr()
+        args.value_cache = self.cache.value_cache[index].data_ptr()
+        _native.check(self.library.tf_prefill_layer(args, self.stream), "prefill_layer")
+        return True
+
+
+def _dense(tensor: Tensor, shape: tuple[int, ...], cache: PagedKVCache) -> bool:
+    return (tensor.shape == shape and tensor.dtype == cache.config.dtype
+            and tensor.device == cache.config.device and tensor.is_contiguous()
+            and tensor.data_ptr() % 16 == 0)
+
+
 def _prefill_packed(weights: DecoderWeights, cache: PagedKVCache, prompts: dict[str, list[int]],
                     ) -> Tensor:
     """Run the packed prefill of reserved, validated prompts; last-position
@@ -614,38 +740,37 @@ def _prefill_packed(weights: DecoderWeights, cache: PagedKVCache, prompts: dict[
     config = weights.config
     hq, hkv, d = config.num_attention_heads, config.num_key_value_heads, config.head_dim
     device = cache.config.device
-    block_size = cache.config.block_size
-    request_ids = list(prompts)
-    lengths = [len(prompts[r]) for r in request_ids]
+    lengths = [len(prompt) for prompt in prompts.values()]
     bounds = np.concatenate(([0], np.cumsum(lengths)))
     total = int(bounds[-1])
-    longs = np.empty((2, total), dtype=np.int64)   # token ids, positions
-    ints = np.ones((3, total), dtype=np.int32)     # pages, offsets, active
-    for i, request_id in enumerate(request_ids):
-        lo, hi = bounds[i], bounds[i + 1]
-        positions = np.arange(hi - lo, dtype=np.int64)
-        pages = np.asarray(cache.page_list(request_id)[0], dtype=np.int32)
-        longs[0, lo:hi] = prompts[request_id]
-        longs[1, lo:hi] = positions
-        ints[0, lo:hi] = pages[positions // block_size]
-        ints[1, lo:hi] = positions % block_size
-    longs_dev = torch.from_numpy(longs).to(device)
-    ints_dev = torch.from_numpy(ints).to(device)
     packed_attention = prefill_attention_supported(weights.embedding.dtype, hq, hkv, d)
-    if packed_attention:
-        tiles = torch.from_numpy(prefill_tiles(lengths)).to(device)
-    tokens, positions_dev = longs_dev[0], longs_dev[1]
+    longs, last, ints, tiles = _stage_prefill(cache, prompts, bounds, prefill_tiles(lengths))
+    positions = longs[1]
     eps = config.rms_norm_eps
-    residual = F.embedding(tokens, weights.embedding)
-    h = rms_norm(residual, weights.layers[0].input_norm, eps)
-    q = torch.empty((total, hq, d), dtype=residual.dtype, device=device)
-    k = torch.empty((total, hkv, d), dtype=residual.dtype, device=device)
-    context = torch.empty((total, hq * d), dtype=residual.dtype, device=device)
+    dtype = weights.embedding.dtype
+    residual = torch.empty((total, config.hidden_size), dtype=dtype, device=device)
+    # The prompts' ids come from the host rows (source -1); the lane state is
+    # not read.
+    residual, h = embedding_rms_norm(longs[0], longs[2], longs[0], weights.embedding,
+                                     weights.layers[0].input_norm, eps, x_output=residual,
+                                     norm_output=torch.empty_like(residual))
+    native = None
+    if _NativePrefill.supported(weights, cache, total):
+        native = _NativePrefill(weights, cache, total, positions, ints, tiles)
+    q = k = context = None
     for index, layer in enumerate(weights.layers):
+        next_norm = (weights.layers[index + 1].input_norm
+                     if index + 1 < len(weights.layers) else weights.final_norm)
+        if native is not None and native.run(index, layer, next_norm, h, residual):
+            continue
+        if context is None:
+            q = torch.empty((total, hq, d), dtype=dtype, device=device)
+            k = torch.empty((total, hkv, d), dtype=dtype, device=device)
+            context = torch.empty((total, hq * d), dtype=dtype, device=device)
         qkv = F.linear(h, layer.qkv)
-        rope_paged_kv_append(qkv, positions_dev, weights.rope_cos, weights.rope_sin,
-                             cache.key_cache[index], cache.value_cache[index], ints_dev[0],
-                             ints_dev[1], ints_dev[2], query_heads=hq, query_output=q,
+        rope_paged_kv_append(qkv, positions, weights.rope_cos, weights.rope_sin,
+                             cache.key_cache[index], cache.value_cache[index], ints[0],
+                             ints[1], ints[2], query_heads=hq, query_output=q,
                              key_output=k)
         if packed_attention:  # every prompt's causal attention in one launch
             prefill_attention(q.view(total, hq * d), k.view(total, hkv * d),
@@ -653,17 +778,17 @@ def _prefill_packed(weights: DecoderWeights, cache: PagedKVCache, prompts: dict[
                               kv_heads=hkv, scale=d ** -0.5, output=context)
         else:
             v = qkv[:, (hq + hkv) * d:].view(total, hkv, d)
-            for i in range(len(request_ids)):
+            for i in range(len(lengths)):
                 lo, hi = int(bounds[i]), int(bounds[i + 1])
                 context[lo:hi] = _causal_attention(q[lo:hi], k[lo:hi], v[lo:hi], d ** -0.5)
         attn = F.linear(context, layer.o_proj)
         residual, h = residual_rms_norm(attn, residual, layer.post_norm, eps)
-        act = swiglu_gate_up(F.linear(h, layer.gate_up))
-        next_norm = (weights.layers[index + 1].input_norm
-                     if index + 1 < len(weights.layers) else weights.final_norm)
+        if prefill_linear_supported(h, layer.gate_up) and layer.gate_up.shape[0] % 16 == 0:
+            act = prefill_linear(h, layer.gate_up, swiglu=True)
+        else:
+            act = swiglu_gate_up(F.linear(h, layer.gate_up))
         residual, h = residual_rms_norm(F.linear(act, layer.down), residual, next_norm, eps)
-    last = torch.from_numpy(bounds[1:] - 1).to(device)
-    return F.linear(h.index_select(0, last), weights.lm_head)
+    return _project(h.index_select(0, last), weights.lm_head)
 
 
 def prefill_requests(weights: DecoderWeights, cache: PagedKVCache,

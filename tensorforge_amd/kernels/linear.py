@@ -298,6 +298,67 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, *, output: Tensor | None = 
     return output
 
 
+def prefill_linear_supported(x: Tensor, weight: Tensor) -> bool:
+    """Whether :func:`prefill_linear` takes these operands (else use F.linear)."""
+
+    return (x.ndim == 2 and weight.ndim == 2 and x.dtype in (torch.float16, torch.bfloat16)
+            and weight.dtype == x.dtype and x.shape[1] == weight.shape[1] and x.shape[1] >= 256
+            and x.shape[1] % 64 == 0 and weight.shape[0] % 8 == 0 and x.stride(1) == 1
+            and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and max(x.stride(0), weight.stride(0)) <= 1 << 21
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.is_cuda
+            and weight.is_cuda)
+
+
+def prefill_linear(x: Tensor, weight: Tensor, *, output: Tensor | None = None, splits: int = 1,
+                   partials: Tensor | None = None, swiglu: bool = False, tile: int = 0) -> Tensor:
+    """``x [m, k] @ weight[n, k].T`` for prefill's packed rows (any m,
+    fp16/bf16, k a multiple of 64): the rounded product in ``output``
+    (allocated when None); with ``partials`` (fp32 ``[splits, m, n]``) the
+    slice sums of ``splits`` slices of K for a consumer that adds them; with
+    ``swiglu`` the activation ``[m, n / 2]`` of a stacked gate|up weight.
+    ``tile`` (0: chosen from the sizes) names the workgroup tile."""
+
+    if not _native.is_available():
+        raise RuntimeError(
+            "the gfx950 kernel library is unavailable; build it with "
+            "`python -m tensorforge_amd.build`"
+        )
+    if not prefill_linear_supported(x, weight):
+        raise ValueError("prefill_linear needs fp16/bf16 CUDA operands [m, k] and [n, k] with k "
+                         ">= 256 a multiple of 64, n of 8, and 16-byte aligned contiguous rows")
+    m, k = x.shape
+    n = weight.shape[0] // 2 if swiglu else weight.shape[0]
+    y_ptr, y_stride, p_ptr = None, 0, None
+    if partials is not None:
+        if swiglu:
+            raise ValueError("the SwiGLU form writes no slice sums")
+        if (partials.shape != (splits, m, n) or partials.dtype != torch.float32
+                or partials.device != x.device or not partials.is_contiguous()):
+            raise ValueError("partials must be a contiguous fp32 [splits, m, n] tensor on x's device")
+        p_ptr = partials.data_ptr()
+        result = partials
+    else:
+        if splits != 1:
+            raise ValueError("several K slices need a partials buffer")
+        if output is None:
+            output = torch.empty((m, n), dtype=x.dtype, device=x.device)
+        if (output.shape != (m, n) or output.dtype != x.dtype or output.device != x.device
+                or output.stride(1) != 1):
+            raise ValueError("output must be [m, n] with contiguous rows, x's dtype and device")
+        y_ptr, y_stride = output.data_ptr(), output.stride(0)
+        result = output
+    _native.check(
+        _native.library().tf_prefill_linear(
+            x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y_ptr, y_stride,
+            p_ptr, m, n, k, splits, int(swiglu), tile, _native.dtype_code(x.dtype),
+            _native.current_stream(x.device),
+        ),
+        "prefill_linear",
+    )
+    return result
+
+
 def linear_partials_sum(partials: Tensor, *, dtype: torch.dtype | None = None,
                         output: Tensor | None = None) -> Tensor:
     """``round(partials.sum(0))`` into fp16/bf16 rows (one rounding)."""
