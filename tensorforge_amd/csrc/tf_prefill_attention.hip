@@ -10,10 +10,10 @@
 //
 // One workgroup of four wavefronts per (block, kv head, group of QH query
 // heads of that kv head); wavefront w serves the block's 16-token tile
-// [b0 + 16 w, +16) for the QH heads.  Each 32-token K/V chunk is loaded once
-// for the workgroup (whole rows, 16 bytes per thread) into one of two LDS
-// buffers while the previous chunk is computed, so a chunk's bytes serve 64
-// query tokens x QH heads instead of the 16 x QH of a wavefront alone.
+// [b0 + 16 w, +16) for the QH heads.  The keys are walked in 64-token
+// chunks that direct-to-LDS loads bring into a ring of buffers (no staging
+// registers or LDS stores), so a chunk's bytes serve 64 query tokens x QH
+// heads and there is one barrier per 64 keys.
 //   scores  v_mfma_f32_16x16x32 with the K chunk (16 tokens x 32 dims per
 //           tile, read from LDS in the A-operand layout) and the head's
 //           query tile as the B operand: lane (l16, q4), register r holds
@@ -22,10 +22,20 @@
 //   P.V     P converted to the storage type is already the B operand; V^T
 //           (A operand) is read from the chunk staged token-major with
 //           ds_read_b64_tr_b16, once per chunk for all QH heads.
-// Softmax in base 2 with a lazily raised running maximum (raised only when a
-// score exceeds it by more than 2^8), fp32 accumulation, one rounding of the
+// The kernel is bound by the softmax's vector work, not by the products: per
+// 16 x 32 scores of a wavefront 8 products (128 cycles at D 64) against some
+// 40 vector instructions, 8 of them exponentials.  So the running maximum is
+// not looked for: the weights are computed against the last one, and only
+// where one of them exceeds 2^8 (which the maximum over the weights, needing
+// no NaN quieting, shows) is the maximum raised and the chunk's weights
+// computed again.  Softmax in base 2, fp32 accumulation, one rounding of the
 // output.
-
+//
+// MI355X: 19 prompts of 8,058 tokens at 32/4 heads, D 64 92.9 -> 57.4 us (613
+// TFLOP/s of causal attention), 4096 + 2051 + 777 tokens at 32/8, D 128 310
+// -> 185 us (958), one prompt of 271 9.2 -> 5.8 us, against 32-key chunks
+// staged through registers with the maximum looked for in every chunk.
+//
 // Reference semantics: the causal scaled-dot-product attention of prefill,
 // tensorforge/runtime/prefill.py:84-88 (causal mask over the padded
 // prompts) and :109-118 (torch SDPA with enable_gqa), here without padding.
@@ -38,11 +48,14 @@ namespace {
 
 constexpr float kPrefillLog2e = 1.4426950408889634f;
 constexpr float kPrefillNegInf = -__builtin_huge_valf();
-constexpr float kPrefillRescale = 8.f;
 constexpr int kPrefillTile = 16;   // query tokens per wavefront
 constexpr int kPrefillWaves = 4;   // wavefronts per workgroup
 constexpr int kPrefillBlock = kPrefillTile * kPrefillWaves;  // query tokens per work item
-constexpr int kPrefillChunk = 32;  // key tokens per step
+constexpr int kPrefillChunk = 64;  // key tokens per LDS buffer
+constexpr float kPrefillFloor = -3e38f;  // running maximum before the first key
+constexpr float kPrefillMost = 256.f;    // weight that makes the maximum rise
+constexpr int kPrefillXcds = 8;
+constexpr int64_t kPrefillPairs = 600;   // workgroups from which a wavefront serves two heads
 
 template <typename T>
 struct PrefillMfma;
@@ -83,8 +96,26 @@ struct PrefillParams {
   float scale_log2;
 };
 
-template <int D>
-constexpr int prefill_row_bytes() { return D * 2 + 16; }
+// 16 bytes per lane from each lane's address straight to LDS at `lds` + 16
+// lane (m0 holds the LDS address; one wait state between its write and the
+// load).  No register is written: vmcnt counts the load, and the LDS bytes
+// are valid after a wait for it.
+__device__ __forceinline__ void prefill_load_lds(const void *src, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "s"(lds)
+      : "memory");
+}
+
+// All but the newest N loads of this wavefront have landed, its LDS reads are
+// done, and so for every wavefront of the workgroup.
+template <int N>
+__device__ __forceinline__ void prefill_wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+}
 
 template <typename T, int D, int QH>
 __global__ void __launch_bounds__(64 * kPrefillWaves)
@@ -93,33 +124,40 @@ prefill_attention_kernel(PrefillParams p) {
   using vec8 = typename M::vec8;
   constexpr int KS = D / 32;
   constexpr int NB = D / 16;
-  constexpr int kRow = prefill_row_bytes<D>();  // V rows (padded for the transpose reads)
-  // K rows are 2 D bytes with their 16-byte pieces permuted: piece p of row r
-  // sits at p ^ ((r / R) % P), P = D / 8 pieces per row, R = 128 / D rows
-  // per 256 bytes (1 at D 128), so the 16 lanes of an A-operand read (rows
-  // 16 j .. +15, one piece each) and the 16 threads of a staging store
-  // cover the 64 banks once.
+  // LDS rows are 2 D bytes with their 16-byte pieces permuted: piece q of row
+  // r sits at q ^ swizzle(r), which changes every R = 128 / D rows (one
+  // 256-byte span of the 64 banks), so the 16 lanes of an operand read (rows
+  // 16 j .. +15, one piece each) cover the banks once.
   constexpr int kPieces = D / 8;
   constexpr int kRowsPer256 = D >= 128 ? 1 : 128 / D;
-  constexpr int kRowK = 2 * D;
-  __shared__ __attribute__((aligned(16))) unsigned char k_lds[2][kPrefillChunk * kRowK];
-  __shared__ __attribute__((aligned(16))) unsigned char v_lds[2][kPrefillChunk * kRow];
-  auto k_offset = [](int row, int piece) {
-    return row * kRowK + 16 * (piece ^ ((row / kRowsPer256) & (kPieces - 1)));
-  };
+  constexpr int kRowBytes = 2 * D;
+  constexpr int kBufBytes = kPrefillChunk * kRowBytes;  // K or V of a chunk
+  constexpr int kStages = D <= 64 ? 3 : 2;
+  constexpr int kSub = D <= 64 ? 64 : 32;  // keys whose operands are held at once
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[kStages][2][kBufBytes];
+  auto swizzle = [](int row) { return (row / kRowsPer256) & (kPieces - 1); };
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int l16 = lane & 15;
   const int q4 = lane >> 4;
-  const int32_t *tile = p.tiles + 3 * static_cast<int64_t>(blockIdx.x);
+  // The blocks come heaviest first, every head group of a block before the
+  // next block.  The dies are dealt workgroups round-robin; where the head
+  // groups are a multiple of the dies, each die takes neighbouring groups,
+  // which share a kv head's K and V in its L2.
+  const int32_t groups = p.group / QH;
+  const int32_t per_block = p.kv_heads * groups;
+  const int32_t block = static_cast<int32_t>(blockIdx.x) / per_block;
+  int32_t hg = static_cast<int32_t>(blockIdx.x) - block * per_block;
+  if (per_block % kPrefillXcds == 0)
+    hg = (hg % kPrefillXcds) * (per_block / kPrefillXcds) + hg / kPrefillXcds;
+  const int32_t *tile = p.tiles + 3 * static_cast<int64_t>(block);
   const int32_t b0 = tile[0];
   const int32_t s = tile[1];
   const int32_t e = tile[2];
-  const int32_t groups = p.group / QH;
-  const int32_t kvh = blockIdx.y / groups;
-  const int32_t h0 = kvh * p.group + (blockIdx.y - kvh * groups) * QH;
+  const int32_t kvh = hg / groups;
+  const int32_t h0 = kvh * p.group + (hg - kvh * groups) * QH;
   // Keys of the block [s, kend_blk); this wavefront's tile [i0, i0 + 16)
   // needs [s, kend) (none when the tile starts past the prompt).
   const int32_t kend_blk = min(b0 + kPrefillBlock, e);
@@ -127,182 +165,192 @@ prefill_attention_kernel(PrefillParams p) {
   const int32_t kend = min(i0 + kPrefillTile, e);
   const int32_t qt = i0 + l16;  // this lane's query token (column)
   const bool q_ok = qt < e;
+  const int32_t nch = (kend_blk - s + kPrefillChunk - 1) / kPrefillChunk;
+  const int32_t my_nch = i0 < e ? (kend - s + kPrefillChunk - 1) / kPrefillChunk : 0;
 
-  const T *qbase = static_cast<const T *>(p.q);
-  const T *kbase = static_cast<const T *>(p.k) + static_cast<int64_t>(kvh) * D;
-  const T *vbase = static_cast<const T *>(p.v) + static_cast<int64_t>(kvh) * D;
+  // Chunk loads: an instruction fills 1024 bytes (kRowsPerLoad rows) of a
+  // buffer; this wavefront's first half are of K, the rest of V.  Rows past
+  // the block's keys read its last key: their scores are masked.
+  constexpr int kLoads = D / 16;  // per wavefront and chunk
+  constexpr int kRowsPerLoad = 1024 / kRowBytes;
+  const int lrow = lane / kPieces;
+  const int64_t strides[2] = {p.k_stride, p.v_stride};
+  const unsigned char *bases[2];
+  bases[0] = reinterpret_cast<const unsigned char *>(static_cast<const T *>(p.k) +
+                                                     static_cast<int64_t>(s) * p.k_stride + static_cast<int64_t>(kvh) * D);
+  bases[1] = reinterpret_cast<const unsigned char *>(static_cast<const T *>(p.v) +
+                                                     static_cast<int64_t>(s) * p.v_stride + static_cast<int64_t>(kvh) * D);
+  int64_t row_off[kLoads];  // bytes of this lane's piece from the chunk's first row
+  auto offset_of = [&](int i, int32_t last) {
+    const int row = kRowsPerLoad * (wave + kPrefillWaves * (i % (kLoads / 2))) + lrow;
+    const int piece = (lane & (kPieces - 1)) ^ swizzle(row);
+    return (static_cast<int64_t>(min(row, last)) * strides[i / (kLoads / 2)]) * 2 + 16 * piece;
+  };
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) row_off[i] = offset_of(i, kPrefillChunk);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char *)&ring[0][0][0]));
+  auto load_chunk = [&](int32_t c, int32_t stage) {
+    const int32_t last = kend_blk - s - kPrefillChunk * c - 1;  // last valid row of the chunk
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int kv = i / (kLoads / 2);
+      const unsigned char *from = bases[kv] + static_cast<int64_t>(kPrefillChunk * c) * strides[kv] * 2;
+      int64_t off = row_off[i];
+      if (last < kPrefillChunk - 1) off = offset_of(i, last);  // uniform
+      const uint32_t at = lds0 + static_cast<uint32_t>((2 * stage + kv) * kBufBytes) +
+                          1024u * static_cast<uint32_t>(wave + kPrefillWaves * (i % (kLoads / 2)));
+      prefill_load_lds(from + off, __builtin_amdgcn_readfirstlane(at));
+    }
+  };
+#pragma unroll
+  for (int c = 0; c < kStages - 1; ++c)
+    if (c < nch) load_chunk(c, c);
 
   vec8 qf[QH][KS];  // B operand: q[token i0 + l16][head h0 + hq][32 ks + 8 q4 .. +8]
   {
-    const T *qrow = qbase + static_cast<int64_t>(q_ok ? qt : s) * p.q_stride;
+    const T *qrow = static_cast<const T *>(p.q) + static_cast<int64_t>(q_ok ? qt : s) * p.q_stride;
 #pragma unroll
     for (int hq = 0; hq < QH; ++hq)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        qf[hq][ks] = q_ok ? *reinterpret_cast<const vec8 *>(qrow + static_cast<int64_t>(h0 + hq) * D +
-                                                            32 * ks + 8 * q4)
-                          : vec8{};
+      for (int ks = 0; ks < KS; ++ks) {
+        const vec8 x = *reinterpret_cast<const vec8 *>(qrow + static_cast<int64_t>(h0 + hq) * D + 32 * ks + 8 * q4);
+        qf[hq][ks] = q_ok ? x : vec8{};
+      }
+  }
+  // LDS offsets of this lane's operand reads within a buffer (rows 16 apart
+  // share their permutation).
+  int k_at[KS], v_at[NB];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) k_at[ks] = l16 * kRowBytes + 16 * ((4 * ks + q4) ^ swizzle(l16));
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const int row = 4 * q4 + (l16 >> 2);
+    v_at[n] = row * kRowBytes + 16 * ((2 * n + ((l16 & 3) >> 1)) ^ swizzle(row)) + 8 * (l16 & 1);
   }
 
   f32x4 acc[QH][NB];
   float m_run[QH], l_run[QH];
 #pragma unroll
   for (int hq = 0; hq < QH; ++hq) {
-    m_run[hq] = kPrefillNegInf;
+    m_run[hq] = kPrefillFloor;
     l_run[hq] = 0.f;
 #pragma unroll
     for (int n = 0; n < NB; ++n) acc[hq][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const int32_t nch = (kend_blk - s + kPrefillChunk - 1) / kPrefillChunk;
-  const int32_t my_nch = i0 < e ? (kend - s + kPrefillChunk - 1) / kPrefillChunk : 0;
 
-  // Staging: the workgroup loads a chunk's K and V rows whole (D / 8
-  // threads of 16 bytes per row) into one of two register sets, two chunks
-  // ahead of the one being computed, and stores them token-major into the
-  // chunk's buffer.  Rows past the block's keys read the prompt's first
-  // row: their V rows are stored as zeros (0 * p), their scores are masked.
-  constexpr int kLanesPerRow = D / 8;
-  constexpr int kRowsPerPass = 64 * kPrefillWaves / kLanesPerRow;
-  constexpr int kPasses = (kPrefillChunk + kRowsPerPass - 1) / kRowsPerPass;
-  const int srow = tid / kLanesPerRow;
-  const int spiece = tid - srow * kLanesPerRow;
-  vec8 kreg[2][kPasses], vreg[2][kPasses];  // register set c % 2 holds chunk c
-  // (the set is a compile-time index: the chunk loop is unrolled by two, so
-  // the sets stay in registers)
-  auto gload = [&](int32_t c, auto set_tag) {
-    constexpr int set = decltype(set_tag)::value;
+  // Keys [t0 + k0, t0 + k0 + kSub) of the chunk at t0.
+  auto compute = [&](int32_t t0, const unsigned char *kb, const unsigned char *vb, int k0) {
+    constexpr int J = kSub / 16;
+    vec8 kf[J][KS];
 #pragma unroll
-    for (int ps = 0; ps < kPasses; ++ps) {
-      const int row = srow + kRowsPerPass * ps;
-      const int32_t t = s + kPrefillChunk * c + row;
-      const int32_t src = (row < kPrefillChunk && t < kend_blk) ? t : s;
-      kreg[set][ps] = *reinterpret_cast<const vec8 *>(kbase + static_cast<int64_t>(src) * p.k_stride + 8 * spiece);
-      vreg[set][ps] = *reinterpret_cast<const vec8 *>(vbase + static_cast<int64_t>(src) * p.v_stride + 8 * spiece);
-    }
-  };
-  auto lstore = [&](int32_t c, auto set_tag) {
-    constexpr int set = decltype(set_tag)::value;
-    unsigned char *kdst = k_lds[set];
-    unsigned char *vdst = v_lds[set];
-    const bool tail = s + kPrefillChunk * (c + 1) > kend_blk;  // uniform
-#pragma unroll
-    for (int ps = 0; ps < kPasses; ++ps) {
-      const int row = srow + kRowsPerPass * ps;
-      if (row < kPrefillChunk) {
-        *reinterpret_cast<vec8 *>(kdst + k_offset(row, spiece)) = kreg[set][ps];
-        vec8 v = vreg[set][ps];
-        if (tail && s + kPrefillChunk * c + row >= kend_blk) v = vec8{};
-        *reinterpret_cast<vec8 *>(vdst + row * kRow + 16 * spiece) = v;
-      }
-    }
-  };
-
-  auto compute = [&](int32_t c, int buf) {
-    const int32_t t0 = s + kPrefillChunk * c;
-    const unsigned char *kb = k_lds[buf];
-    const unsigned char *vb = v_lds[buf];
-    // K in the A-operand layout: lane (l16, q4) of tile j holds token
-    // t0 + 16 j + l16, dims [32 ks + 8 q4, +8).
-    vec8 kf[2][KS];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
-        kf[j][ks] = *reinterpret_cast<const vec8 *>(kb + k_offset(16 * j + l16, 4 * ks + q4));
-    // V^T once for all heads.
-    vec8 vtf[NB];
-    {
-      const unsigned char *rd = vb + (4 * q4 + (l16 >> 2)) * kRow + (l16 & 3) * 8;
+        kf[j][ks] = *reinterpret_cast<const vec8 *>(kb + k_at[ks] + (k0 + 16 * j) * kRowBytes);
+    // Causal mask: needed when some key of the step lies past the tile's
+    // first query token (a query's own token bounds its keys in the prompt).
+    const bool masked = t0 + k0 + kSub - 1 > i0;
+    const int32_t limit = qt - t0 - k0 - 4 * q4;  // key 16 j + r (of q4 = 0) is seen up to this
+    vec8 pf[QH][J / 2];
+    // Every head's scores and weights before any of the rare paths below, so
+    // the heads' products and exponentials interleave.
+    float sc[QH][4 * J], pr[QH][4 * J];
 #pragma unroll
-      for (int n = 0; n < NB; ++n) {
-        const pf_i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4 *)(rd + 32 * n));
-        const pf_i16x4 hi =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4 *)(rd + 16 * kRow + 32 * n));
-        vtf[n] = __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      }
-    }
-    // Causal mask: needed when some key token of the chunk lies past the
-    // tile's first query token or past the tile's keys.
-    const bool masked = t0 + kPrefillChunk > kend || t0 + kPrefillChunk - 1 > i0;
+    for (int hq = 0; hq < QH; ++hq)
 #pragma unroll
-    for (int hq = 0; hq < QH; ++hq) {
-      float sc[8];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < J; ++j) {
         f32x4 acc_s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) acc_s = M::mma(kf[j][ks], qf[hq][ks], acc_s);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[4 * j + r] = acc_s[r];
+        for (int r = 0; r < 4; ++r) sc[hq][4 * j + r] = acc_s[r];
       }
-      if (masked) {
+    if (masked) {
+      int32_t seen = limit;
+      asm volatile("" : "+v"(seen));  // keeps the comparisons inside the branch
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < J; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int32_t kt = t0 + 16 * j + 4 * q4 + r;
-            if (kt >= kend || kt > qt) sc[4 * j + r] = kPrefillNegInf;
-          }
-      }
-      float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])),
-                       fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-      mx *= p.scale_log2;
-      if (__ballot(mx > m_run[hq] + kPrefillRescale) != 0) {
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int hq = 0; hq < QH; ++hq)
+            if (16 * j + r > seen) sc[hq][4 * j + r] = kPrefillNegInf;
+    }
+    auto weights = [&](int hq) {
+#pragma unroll
+      for (int i = 0; i < 4 * J; ++i)
+        pr[hq][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[hq][i], p.scale_log2, -m_run[hq]));
+    };
+    float top = 0.f;
+#pragma unroll
+    for (int hq = 0; hq < QH; ++hq) {
+      weights(hq);
+#pragma unroll
+      for (int i = 0; i < 4 * J; i += 2) top = fmaxf(fmaxf(pr[hq][i], pr[hq][i + 1]), top);
+    }
+    if (__ballot(top > kPrefillMost) != 0) {  // uniform: raise the maxima
+#pragma unroll
+      for (int hq = 0; hq < QH; ++hq) {
+        float mx = sc[hq][0] * p.scale_log2;
+#pragma unroll
+        for (int i = 1; i < 4 * J; ++i) mx = fmaxf(mx, sc[hq][i] * p.scale_log2);
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         const float m_new = fmaxf(m_run[hq], mx);
-        // A column whose keys are all masked so far keeps m = -inf.
-        const float alpha = m_new == kPrefillNegInf ? 1.f : __builtin_amdgcn_exp2f(m_run[hq] - m_new);
+        const float alpha = __builtin_amdgcn_exp2f(m_run[hq] - m_new);
         m_run[hq] = m_new;
         l_run[hq] *= alpha;
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[hq][n] *= alpha;
+        weights(hq);
       }
-      // m_run is finite here: every query column sees its prompt's first
-      // key (token s <= the query) in chunk 0, whose scores raise it from
-      // -inf; masked scores give weights exp2(-inf) = 0.
-      vec8 pf;
-      float psum = 0.f;
+    }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], p.scale_log2, -m_run[hq]));
-        psum += pr;
-        pf[i] = static_cast<T>(pr);
+    for (int hq = 0; hq < QH; ++hq) {
+      float sum[4] = {pr[hq][0], pr[hq][1], pr[hq][2], pr[hq][3]};
+#pragma unroll
+      for (int i = 0; i < 4 * J; ++i) {
+        if (i >= 4) sum[i & 3] += pr[hq][i];
+        pf[hq][i >> 3][i & 7] = static_cast<T>(pr[hq][i]);
       }
-      l_run[hq] += psum;
+      l_run[hq] += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    }
 #pragma unroll
-      for (int n = 0; n < NB; ++n) acc[hq][n] = M::mma(vtf[n], pf, acc[hq][n]);
+    for (int h = 0; h < J / 2; ++h) {
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        const unsigned char *rd = vb + v_at[n] + (k0 + 32 * h) * kRowBytes;
+        const pf_i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4 *)rd);
+        const pf_i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4 *)(rd + 16 * kRowBytes));
+        const vec8 vt = __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int hq = 0; hq < QH; ++hq) acc[hq][n] = M::mma(vt, pf[hq][h], acc[hq][n]);
+      }
     }
   };
 
-  // Chunk c is computed from buffer c % 2 while the loads of chunks c + 1
-  // and c + 2 are in flight; after it, chunk c + 1 is stored into the other
-  // buffer (last read for chunk c - 1, before the previous barrier) and the
-  // loads of c + 3 are issued into the register set c + 1 freed.  One
-  // barrier per chunk publishes the stored buffer and retires the one just
-  // read.
-  using Set0 = std::integral_constant<int, 0>;
-  using Set1 = std::integral_constant<int, 1>;
-  gload(0, Set0{});
-  if (nch > 1) gload(1, Set1{});
-  lstore(0, Set0{});
-  if (nch > 2) gload(2, Set0{});
-  __syncthreads();
-  for (int32_t c = 0; c < nch; c += 2) {
-    // even chunk c: buffer and register set 0; then chunk c + 1 (set 1)
-    if (c < my_nch) compute(c, 0);  // wavefront-uniform
-    if (c + 1 < nch) {
-      lstore(c + 1, Set1{});
-      if (c + 3 < nch) gload(c + 3, Set1{});
+  // Chunk c waits for its own loads (the next chunk's may stay in flight);
+  // past the barrier every wavefront is done with chunk c - 1, whose buffer
+  // takes chunk c + kStages - 1.
+  int32_t stage = 0;
+  for (int32_t c = 0; c < nch; ++c) {
+    if (kStages > 2 && c + 1 < nch)
+      prefill_wait_barrier<(kStages - 2) * kLoads>();
+    else
+      prefill_wait_barrier<0>();
+    if (c + kStages - 1 < nch) load_chunk(c + kStages - 1, stage == 0 ? kStages - 1 : stage - 1);
+    if (c < my_nch) {  // wavefront-uniform
+      const unsigned char *kb = ring[stage][0];
+      const unsigned char *vb = ring[stage][1];
+#pragma unroll
+      for (int k0 = 0; k0 < kPrefillChunk; k0 += kSub) {
+        // The second half of a chunk past the tile's keys has nothing to add.
+        if (k0 > 0 && s + kPrefillChunk * c + k0 >= kend) break;
+        compute(s + kPrefillChunk * c, kb, vb, k0);
+      }
     }
-    __syncthreads();
-    if (c + 1 >= nch) break;
-    if (c + 1 < my_nch) compute(c + 1, 1);
-    if (c + 2 < nch) {
-      lstore(c + 2, Set0{});
-      if (c + 4 < nch) gload(c + 4, Set0{});
-    }
-    __syncthreads();
+    stage = stage + 1 == kStages ? 0 : stage + 1;
   }
 
   // Lane-partial sums -> per-column sums; write the query tokens of the prompt.
@@ -327,9 +375,8 @@ prefill_attention_kernel(PrefillParams p) {
 
 template <typename T, int D, int QH>
 void launch_prefill(const PrefillParams &p, int32_t ntiles, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(ntiles),
-                  static_cast<unsigned>(p.kv_heads * (p.group / QH)));
-  hipLaunchKernelGGL((prefill_attention_kernel<T, D, QH>), grid, dim3(64 * kPrefillWaves), 0,
+  const unsigned grid = static_cast<unsigned>(ntiles) * static_cast<unsigned>(p.kv_heads * (p.group / QH));
+  hipLaunchKernelGGL((prefill_attention_kernel<T, D, QH>), dim3(grid), dim3(64 * kPrefillWaves), 0,
                      stream, p);
 }
 
@@ -337,12 +384,17 @@ template <typename T, int D>
 void launch_prefill_qh(const PrefillParams &p, int32_t ntiles, int32_t heads_per_wave,
                        hipStream_t stream) {
   // Query heads per wavefront (a power of two dividing the group): as asked,
-  // else 2 at head_dim >= 64 and 1 at 32 (measured best on MI355X over a
-  // cfg5 batch of 19 prompts, 8,058 tokens: 97.5 / 102.1 / 111.8 us for 2 /
-  // 1 / 4 at D 64, 165 / 165 / 199 at D 128, 39.8 / 47.0 for 1 / 2 at D 32);
-  // at most 4 at head_dim 128, for registers.
+  // else one at head_dim 32 and wherever two would leave fewer than
+  // kPrefillPairs workgroups -- a call then waits for its longest chain of
+  // chunks, which one head shortens -- and two otherwise, which read each
+  // chunk's operands half as often (MI355X, us with one / two heads: 271
+  // tokens 5.8 / 7.4, 2048 30.4 / 34.4, 3 x 1000 25.9 / 24.3, 19 prompts of
+  // 8,058 tokens 71.6 / 57.4 at 32/4 heads, D 64; 2048 53.7 / 52.2, 4096 +
+  // 2051 + 777 249 / 185 at 32/8, D 128; 19.6 / 24.9 at 8/2, D 32).  At most
+  // 4 at head_dim 128, for registers.
   constexpr int kMax = D >= 128 ? 4 : 8;
-  int32_t qh = heads_per_wave > 0 ? heads_per_wave : (D >= 64 ? 2 : 1);
+  const int64_t pairs = static_cast<int64_t>(ntiles) * p.kv_heads * ((p.group + 1) / 2);
+  int32_t qh = heads_per_wave > 0 ? heads_per_wave : (D >= 64 && pairs >= kPrefillPairs ? 2 : 1);
   if (qh > kMax) qh = kMax;
   if (qh > p.group) qh = p.group;
   switch (qh) {
