@@ -14,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -21,6 +22,8 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 SOURCE_DIR = PACKAGE_DIR / "csrc"
 LIBRARY_DIR = PACKAGE_DIR / "lib"
 LIBRARY_PATH = LIBRARY_DIR / "libtensorforge_amd.so"
+BINDING_SOURCE = SOURCE_DIR / "tf_python.cpp"
+BINDING_PATH = LIBRARY_DIR / "_tf_launch.so"
 BUILD_DIR = PACKAGE_DIR.parent / "_build"
 ARCH = "gfx950"
 
@@ -72,8 +75,25 @@ def _compile(source: Path, compiler: str) -> Path:
     return obj
 
 
+def _build_binding() -> None:
+    """The CPython module that calls the library (host code only), linked to
+    it by its place beside it."""
+
+    compiler = shutil.which("g++") or "g++"
+    tmp = BINDING_PATH.with_suffix(".so.tmp")
+    cmd = [compiler, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-I{sysconfig.get_paths()['include']}", str(BINDING_SOURCE), "-o", str(tmp),
+           f"-L{LIBRARY_DIR}", "-ltensorforge_amd", "-Wl,-rpath,$ORIGIN",
+           "-Wl,--allow-shlib-undefined"]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"g++ failed for {BINDING_SOURCE.name}:\n{result.stderr}")
+    os.replace(tmp, BINDING_PATH)
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile all kernels for gfx950 and link the shared library."""
+    """Compile all kernels for gfx950, link the shared library and build its
+    Python binding."""
 
     compiler = hipcc()
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
@@ -98,6 +118,7 @@ def build(verbose: bool = False) -> Path:
     if result.returncode != 0:
         raise RuntimeError(f"link failed:\n{result.stderr}")
     os.replace(tmp, LIBRARY_PATH)
+    _build_binding()
     if verbose:
         print(f"built {LIBRARY_PATH}")
     return LIBRARY_PATH

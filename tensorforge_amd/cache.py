@@ -260,7 +260,7 @@ class PagedKVCache:
         value_layer = self.value_cache[layer_index]
         table = self.block_tables[sequence.slot]
         _native.check(
-            _native.library().tf_paged_kv_write_range(
+            _native.launch().tf_paged_kv_write_range(
                 keys.data_ptr(), values.data_ptr(), key_layer.data_ptr(), value_layer.data_ptr(),
                 table.data_ptr(), table.numel(), reservation.start_position,
                 reservation.token_count, self.config.num_kv_heads, self.config.head_dim,

@@ -38,6 +38,7 @@ initialize_weights (layers.py:174-176).
 
 from __future__ import annotations
 
+import ctypes
 import time
 from collections.abc import Callable
 from contextlib import suppress
@@ -660,7 +661,7 @@ class _NativePrefill:
         hq, hkv, d = config.num_attention_heads, config.num_key_value_heads, config.head_dim
         hidden, inter = config.hidden_size, config.intermediate_size
         self.cache = cache
-        self.library = _native.library()
+        self.library = _native.launch()
         self.stream = _native.current_stream(cache.config.device)
         qkv_width = (hq + 2 * hkv) * d
         self.shapes = {"qkv": (qkv_width, hidden), "o_proj": (hidden, hq * d),
@@ -684,6 +685,7 @@ class _NativePrefill:
             hidden=hidden, intermediate=inter, query_heads=hq, kv_heads=hkv, head_dim=d,
             num_blocks=cache.config.num_blocks, block_size=cache.config.block_size,
             eps=config.rms_norm_eps, scale=d ** -0.5, dtype=_native.dtype_code(dtype))
+        self.address = ctypes.addressof(self.args)
 
     @staticmethod
     def supported(weights: DecoderWeights, cache: PagedKVCache, total: int) -> bool:
@@ -721,7 +723,7 @@ class _NativePrefill:
         args.next_norm = next_norm.data_ptr()
         args.key_cache = self.cache.key_cache[index].data_ptr()
         args.value_cache = self.cache.value_cache[index].data_ptr()
-        _native.check(self.library.tf_prefill_layer(args, self.stream), "prefill_layer")
+        _native.check(self.library.tf_prefill_layer(self.address, self.stream), "prefill_layer")
         return True
 
 

@@ -13,6 +13,7 @@ torch's current stream; nothing here synchronises with the device when
 from __future__ import annotations
 
 import dataclasses
+import functools
 from dataclasses import dataclass
 from typing import Any
 
@@ -406,6 +407,26 @@ def attention_plan(launch_context: int, batch: int, kv_heads: int, context_capac
     return split if split is not None else one_pass
 
 
+@functools.lru_cache(maxsize=4096)
+def _plan_for(fixed_split: int | None, generic: bool, launch_context: int, batch: int,
+              kv_heads: int, context_capacity: int, attention_path: str, slot_limit: int,
+              head_dim: int, element_bytes: int) -> tuple[AttentionPlan, int]:
+    """The plan of a call and its launch flags, a function of sizes alone
+    (``fixed_split`` is the caller-fixed partition size :func:`attention_plan`
+    reads); ``generic``: for the generic kernel, which takes fixed partitions
+    and no launch flags beyond them."""
+
+    plan = attention_plan(launch_context, batch, kv_heads, context_capacity, attention_path,
+                          slot_limit, head_dim=head_dim, element_bytes=element_bytes)
+    if plan.balanced and generic:
+        # Fixed partitions sized for about one workgroup per compute unit like
+        # any narrow call's (4 rows of 8192 at 32/8 heads, D 128, fp32: 56 us
+        # in partitions of 1024 tokens against 173 in the balanced plan's 64).
+        fixed = narrow_split_plan(launch_context, batch, kv_heads, head_dim, element_bytes, slot_limit)
+        plan = fixed if fixed is not None else dataclasses.replace(plan, balanced=False, heads_per_wg=1)
+    return plan, plan.flags
+
+
 def paged_gqa_decode_attention(
     query: Tensor,
     key_cache: Tensor,
@@ -494,21 +515,13 @@ def paged_gqa_decode_attention(
                          workspace.partial_accumulator.shape[0]) // max(batch * query_heads, 1)
     else:
         slot_limit = COMPUTE_UNITS * BALANCED_MAX_HEADS_PER_WG
-    plan = attention_plan(launch_context, batch, kv_heads, context_capacity, attention_path,
-                          slot_limit, head_dim=head_dim, element_bytes=query.element_size())
     dtype = _native.dtype_code(query.dtype)
     group = query_heads // kv_heads
-    variant = _native.library().tf_paged_gqa_decode_variant(dtype, head_dim, group, block_size, 0)
+    variant = _native.launch().tf_paged_gqa_decode_variant(dtype, head_dim, group, block_size, 0)
     kernel = "mfma" if variant == _native.TF_ATTENTION_MFMA else "generic"
-    if plan.balanced and kernel != "mfma":
-        # The generic kernel takes fixed partitions, sized for about one
-        # workgroup per compute unit like any narrow call's (4 rows of 8192
-        # at 32/8 heads, D 128, fp32: 56 us in partitions of 1024 tokens
-        # against 173 in the balanced plan's 64).
-        fixed = narrow_split_plan(launch_context, batch, kv_heads, head_dim,
-                                  query.element_size(), slot_limit)
-        plan = fixed if fixed is not None else dataclasses.replace(
-            plan, balanced=False, heads_per_wg=1)
+    plan, flags = _plan_for(_SPLIT_SIZE, kernel != "mfma", launch_context, batch, kv_heads,
+                            context_capacity, attention_path, slot_limit, head_dim,
+                            query.element_size())
     use_split_kv = not plan.one_pass
     split_size = plan.split_size
     device = query.device
@@ -551,7 +564,7 @@ def paged_gqa_decode_attention(
         # counters enable (the C ABI keeps both).
         counters_ptr = None
         _native.check(
-            _native.library().tf_paged_gqa_decode(
+            _native.launch().tf_paged_gqa_decode(
                 query.data_ptr(),
                 key_cache.data_ptr(),
                 value_cache.data_ptr(),
@@ -575,7 +588,7 @@ def paged_gqa_decode_attention(
                 num_splits,
                 attention_scale,
                 dtype,
-                plan.flags,
+                flags,
                 stream,
             ),
             "paged_gqa_decode_attention",
@@ -595,7 +608,7 @@ def paged_gqa_decode_attention(
         one_pass_size = plan.split_size
         num_splits = 1
         _native.check(
-            _native.library().tf_paged_gqa_decode(
+            _native.launch().tf_paged_gqa_decode(
                 query.data_ptr(),
                 key_cache.data_ptr(),
                 value_cache.data_ptr(),
@@ -619,7 +632,7 @@ def paged_gqa_decode_attention(
                 1,
                 attention_scale,
                 dtype,
-                plan.flags,
+                flags,
                 stream,
             ),
             "paged_gqa_decode_attention",
@@ -716,16 +729,16 @@ def paged_gqa_decode_attention_rope_append(
         raise ValueError("max_context_length must be positive and within table capacity")
     capacity = min(workspace.partial_max.numel(), workspace.partial_sum.numel(),
                    workspace.partial_accumulator.shape[0])
-    plan = attention_plan(max_context_length, batch, kv_heads, context_capacity,
-                          slot_limit=capacity // max(batch * query_heads, 1), head_dim=head_dim,
-                          element_bytes=qkv.element_size())
+    plan, flags = _plan_for(_SPLIT_SIZE, False, max_context_length, batch, kv_heads,
+                            context_capacity, "auto", capacity // max(batch * query_heads, 1),
+                            head_dim, qkv.element_size())
     head_bucket = _next_power_of_2(head_dim)
     partial_programs = batch * query_heads * plan.num_splits
     if not plan.one_pass and (capacity < partial_programs
                               or workspace.partial_accumulator.shape[1] != head_bucket):
         raise ValueError("split-KV workspace has insufficient or incompatible capacity")
     _native.check(
-        _native.library().tf_paged_gqa_decode_rope_append(
+        _native.launch().tf_paged_gqa_decode_rope_append(
             qkv.data_ptr(), qkv.stride(0), positions.data_ptr(), cos_table.data_ptr(),
             sin_table.data_ptr(), cos_table.shape[0], key_cache.data_ptr(),
             value_cache.data_ptr(), append_pages.data_ptr(), append_offsets.data_ptr(),
@@ -734,7 +747,7 @@ def paged_gqa_decode_attention_rope_append(
             workspace.partial_accumulator.data_ptr(), None, capacity, head_bucket, batch,
             query_heads, kv_heads, head_dim, num_blocks, block_size, table_width,
             plan.split_size, plan.num_splits, head_dim**-0.5 if scale is None else scale,
-            _native.dtype_code(qkv.dtype), plan.flags, _native.current_stream(qkv.device),
+            _native.dtype_code(qkv.dtype), flags, _native.current_stream(qkv.device),
         ),
         "paged_gqa_decode_attention_rope_append",
     )

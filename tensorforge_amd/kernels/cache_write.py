@@ -73,7 +73,7 @@ def paged_kv_write_token(
             raise ValueError(f"{name} must be int32 with shape [batch]")
     num_blocks, block_size, kv_heads, head_dim = key_cache.shape
     _native.check(
-        _native.library().tf_paged_kv_write_token(
+        _native.launch().tf_paged_kv_write_token(
             keys.data_ptr(),
             values.data_ptr(),
             key_cache.data_ptr(),
@@ -136,7 +136,7 @@ def paged_kv_write_slots(
         raise ValueError("slot_mapping must be int64 with shape [tokens]")
     num_blocks, block_size, kv_heads, head_dim = key_cache.shape
     _native.check(
-        _native.library().tf_paged_kv_write_slots(
+        _native.launch().tf_paged_kv_write_slots(
             keys.data_ptr(),
             values.data_ptr(),
             key_cache.data_ptr(),

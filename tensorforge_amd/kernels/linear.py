@@ -63,7 +63,7 @@ def linear_rows(x: Tensor, weight: Tensor, *, output: Tensor | None = None,
             or output.stride(1) != 1):
         raise ValueError("output must be [m, n] with contiguous rows, x's dtype and device")
     _native.check(
-        _native.library().tf_linear_rows(
+        _native.launch().tf_linear_rows(
             x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), output.data_ptr(),
             output.stride(0), m, n, k, waves_per_tile, _native.dtype_code(x.dtype),
             _native.current_stream(x.device),
@@ -114,7 +114,7 @@ def linear_partials(x: Tensor, weight: Tensor, splits: int, *,
             or partials.device != x.device or not partials.is_contiguous()):
         raise ValueError("partials must be a contiguous fp32 [splits, m, n] tensor on x's device")
     _native.check(
-        _native.library().tf_linear_partials(
+        _native.launch().tf_linear_partials(
             x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), partials.data_ptr(),
             m, n, k, splits, _native.dtype_code(x.dtype), _native.current_stream(x.device),
         ),
@@ -159,7 +159,7 @@ def linear_stream(x: Tensor, weight: Tensor, *, splits: int = 1, output: Tensor 
         y_ptr, y_stride = output.data_ptr(), output.stride(0)
         result = output
     _native.check(
-        _native.library().tf_linear_stream(
+        _native.launch().tf_linear_stream(
             x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y_ptr, y_stride,
             p_ptr, m, n, k, splits, _native.dtype_code(x.dtype), _native.current_stream(x.device),
         ),
@@ -203,7 +203,7 @@ def linear_kstream(x: Tensor, weight: Tensor, *, output: Tensor | None = None,
     if (output.shape != (m, n) or output.dtype != x.dtype or output.device != x.device
             or output.stride(1) != 1):
         raise ValueError("output must be [m, n] with contiguous rows, x's dtype and device")
-    library = _native.library()
+    library = _native.launch()
     stream = _native.current_stream(x.device)
     if residual is not None:
         if (residual.shape != (m, n) or residual.dtype != x.dtype
@@ -279,7 +279,7 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, *, output: Tensor | None = 
     if (output.shape != (m, inter) or output.dtype != x.dtype or output.device != x.device
             or output.stride(1) != 1):
         raise ValueError("output must be [m, I] with contiguous rows, x's dtype and device")
-    library = _native.library()
+    library = _native.launch()
     args = (x.data_ptr(), x.stride(0), gate_up_weight.data_ptr(), gate_up_weight.stride(0),
             output.data_ptr(), output.stride(0), m, inter, k)
     if norm_eps is not None:
@@ -349,7 +349,7 @@ def prefill_linear(x: Tensor, weight: Tensor, *, output: Tensor | None = None, s
         y_ptr, y_stride = output.data_ptr(), output.stride(0)
         result = output
     _native.check(
-        _native.library().tf_prefill_linear(
+        _native.launch().tf_prefill_linear(
             x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y_ptr, y_stride,
             p_ptr, m, n, k, splits, int(swiglu), tile, _native.dtype_code(x.dtype),
             _native.current_stream(x.device),
@@ -372,7 +372,7 @@ def linear_partials_sum(partials: Tensor, *, dtype: torch.dtype | None = None,
             or output.dtype not in (torch.float16, torch.bfloat16)):
         raise ValueError("output must be fp16/bf16 [m, n] with contiguous rows on the same device")
     _native.check(
-        _native.library().tf_linear_partials_sum(
+        _native.launch().tf_linear_partials_sum(
             partials.data_ptr(), splits, m, n, output.data_ptr(), output.stride(0),
             _native.dtype_code(output.dtype), _native.current_stream(partials.device),
         ),

@@ -85,7 +85,7 @@ def _norm_config(columns: int, dtype: torch.dtype, aligned: bool,
     reference's autotune set, triton_ops.py:28-33) that leave each lane at
     most ``per_lane`` vectors (1 when summing split-K partials)."""
 
-    vector = 16 // torch.empty((), dtype=dtype).element_size()
+    vector = 4 if dtype == torch.float32 else 8
     vectorised = aligned and columns % vector == 0
     width = vector if vectorised else 1
     units = columns // width
@@ -140,7 +140,7 @@ def embedding_rms_norm(
                 or t.device != embedding.device):
             raise ValueError(f"{name} must be a contiguous [rows, hidden] tensor like the table")
     _native.check(
-        _native.library().tf_embedding_rms_norm(
+        _native.launch().tf_embedding_rms_norm(
             token_state.data_ptr(), token_state.shape[0], source_lanes.data_ptr(),
             host_tokens.data_ptr(), embedding.data_ptr(), vocab, weight.data_ptr(),
             x_output.data_ptr(), norm_output.data_ptr(), rows, columns, eps,
@@ -167,7 +167,7 @@ def rms_norm(
     rows, columns = _norm_launch_shape(inputs)
     output = _output_or_empty(output, inputs, "output")
     _native.check(
-        _native.library().tf_rms_norm(
+        _native.launch().tf_rms_norm(
             inputs.data_ptr(),
             weight.data_ptr(),
             output.data_ptr(),
@@ -215,7 +215,7 @@ def residual_rms_norm(
     residual_output = _output_or_empty(residual_output, inputs, "residual_output")
     norm_output = _output_or_empty(norm_output, inputs, "norm_output")
     _native.check(
-        _native.library().tf_residual_rms_norm(
+        _native.launch().tf_residual_rms_norm(
             inputs.data_ptr(),
             residual.data_ptr(),
             weight.data_ptr(),
@@ -269,7 +269,7 @@ def residual_rms_norm_partials(
     residual_output = _output_or_empty(residual_output, residual, "residual_output")
     norm_output = _output_or_empty(norm_output, residual, "norm_output")
     _native.check(
-        _native.library().tf_residual_rms_norm_partials(
+        _native.launch().tf_residual_rms_norm_partials(
             partials.data_ptr(),
             partials.shape[0],
             residual.data_ptr(),
@@ -298,7 +298,7 @@ def swiglu(gate: Tensor, up: Tensor, *, output: Tensor | None = None) -> Tensor:
     output = _output_or_empty(output, gate, "output")
     numel = gate.numel()
     _native.check(
-        _native.library().tf_swiglu(
+        _native.launch().tf_swiglu(
             gate.data_ptr(),
             up.data_ptr(),
             output.data_ptr(),
@@ -344,7 +344,7 @@ def swiglu_gate_up(gate_up: Tensor, *, output: Tensor | None = None) -> Tensor:
             or output.device != gate_up.device or output.stride(1) != 1):
         raise ValueError("output must be [rows, F] with contiguous rows, gate_up's dtype and device")
     _native.check(
-        _native.library().tf_swiglu_rows(
+        _native.launch().tf_swiglu_rows(
             gate_up.data_ptr(), gate_up.stride(0), output.data_ptr(), output.stride(0), rows,
             columns, _native.dtype_code(gate_up.dtype), _native.current_stream(gate_up.device),
         ),
@@ -376,7 +376,7 @@ def argmax_rows(logits: Tensor, *, output: Tensor | None = None) -> Tensor:
             or (rows > 1 and output.stride(0) != 1)):
         raise ValueError("output must be a contiguous int64 [rows] tensor on the logits' device")
     _native.check(
-        _native.library().tf_argmax_rows(
+        _native.launch().tf_argmax_rows(
             logits.data_ptr(), logits.stride(0) if rows > 1 else columns, rows, columns,
             _native.dtype_code(logits.dtype), output.data_ptr(),
             _native.current_stream(logits.device),

@@ -79,7 +79,7 @@ def prefill_attention(q: Tensor, k: Tensor, v: Tensor, tiles: Tensor, *, query_h
     if tiles.dtype != torch.int32 or tiles.ndim != 2 or tiles.shape[1] != 3 or not tiles.is_cuda:
         raise ValueError("tiles must be a CUDA int32 [n, 3] tensor from prefill_tiles")
     _native.check(
-        _native.library().tf_prefill_attention(
+        _native.launch().tf_prefill_attention(
             q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
             output.data_ptr(), output.stride(0), tiles.data_ptr(), tiles.shape[0], query_heads,
             kv_heads, head_dim, scale, heads_per_wave, _native.dtype_code(q.dtype),

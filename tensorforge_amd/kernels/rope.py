@@ -86,7 +86,7 @@ def rope_paged_kv_append(
         if tensor.shape != (batch,) or tensor.dtype != torch.int32:
             raise ValueError(f"{name} must be int32 with shape [batch]")
     _native.check(
-        _native.library().tf_rope_kv_append(
+        _native.launch().tf_rope_kv_append(
             qkv.data_ptr(), qkv.stride(0), positions.data_ptr(), cos_table.data_ptr(),
             sin_table.data_ptr(), cos_table.shape[0], query_output.data_ptr(),
             None if key_output is None else key_output.data_ptr(), key_cache.data_ptr(),
