@@ -37,8 +37,8 @@
  *   tf_linear_partials_sum   K into fp32 partials and their row sum
  *   tf_linear_stream         the same projections staged through LDS with
  *                            whole-row loads (direct or split-K partials)
- *   tf_linear_kstream        the same projections, K split over a 16-column
- *                            workgroup's wavefronts (narrow weights)
+ *   tf_linear_kstream        the same projections, K split over a workgroup's
+ *                            wavefronts (a decode step's projections)
  *   tf_linear_kswiglu        its K-split form
  *   tf_linear_kstream_norm,  the same K-split projections fused with the
  *   tf_linear_kswiglu_norm   RMSNorm before them (triton_ops.py:179-205)
@@ -447,9 +447,9 @@ int32_t tf_linear_stream(const void *x, int64_t x_row_stride, const void *weight
 
 /*
  * y = round(x @ weight^T) for up to 64 rows with K split over the four
- * wavefronts of a 16-column workgroup, each staging its k chunks of x and
- * weight through LDS with whole-row loads: the form for weights with few
- * 64-column tiles (a 2560-row qkv projection).  K % 32 == 0, 16-byte aligned
+ * wavefronts of a workgroup, each loading its k chunks of x and weight
+ * straight to LDS.  The tile follows the sizes and changes no bit of a
+ * row's result.  K % 32 == 0, 16-byte aligned
  * x and weight rows, fp16/bf16.  Replaces the torch GEMM of the decode
  * projections (tensorforge/model/layers.py:88-95) as the decode step calls
  * them (tensorforge/runtime/decode_bucket.py:441-447).
@@ -461,8 +461,7 @@ int32_t tf_linear_kstream(const void *x, int64_t x_row_stride, const void *weigh
 /*
  * tf_linear_swiglu's result (the stacked gate|up projection and its SwiGLU,
  * bit for bit tf_linear_kstream of the stacked weight followed by
- * tf_swiglu_rows) with K split over the four wavefronts of a workgroup of
- * 16 activation columns: the form for 33..64 rows, where x is large.
+ * tf_swiglu_rows) with K split over the four wavefronts of a workgroup.
  */
 int32_t tf_linear_kswiglu(const void *x, int64_t x_row_stride, const void *gate_up_weight,
                           int64_t weight_row_stride, void *y, int64_t y_row_stride, int32_t m,
@@ -487,10 +486,7 @@ int32_t tf_linear_kstream_norm(const void *x, int64_t x_row_stride, const void *
  * scaled by rsqrt(mean_k(x[i][k]^2) + eps) before the activation, the
  * stacked weight carrying the norm's gain.  Replaces the reference's
  * post-attention RMSNorm followed by the MLP's gate and up projections and
- * SwiGLU (triton_ops.py:179-205; model/layers.py:144-158).  At 49-64 rows
- * with k = 2048 (and 2048-8192 intermediate columns) the launch keeps each
- * workgroup's 32 rows of x in LDS and streams only the weight; the results
- * are the same bits either way.
+ * SwiGLU (triton_ops.py:179-205; model/layers.py:144-158).
  */
 int32_t tf_linear_kswiglu_norm(const void *x, int64_t x_row_stride, const void *gate_up_weight,
                                int64_t weight_row_stride, void *y, int64_t y_row_stride, int32_t m,

@@ -41,6 +41,7 @@
 #include "tf_common.hpp"
 
 #include <atomic>
+#include <type_traits>
 
 namespace tf {
 namespace {
@@ -319,27 +320,30 @@ linear_stream_kernel(const T *__restrict__ x, int64_t x_stride, const T *__restr
 }
 
 // ---------------------------------------------------------------------------
-// K-split form of the weight stream for narrow weights (few 64-column tiles,
-// e.g. a 2560-row qkv projection) and for the gate|up + SwiGLU launch: a
-// workgroup owns NT 16-column tiles over all of K and its four wavefronts
-// take a quarter of K each.  Every wavefront stages its own KC-wide k
-// chunks of x (16 MT rows) and of its weight rows in a private LDS region
-// with whole-row loads (KC / 8 lanes per row piece), so the x re-reads (once
-// per workgroup) run at the L2 rate of whole-line loads, and the four
-// tiles meet once in LDS.  Each x operand read from LDS feeds NT (twice NT
-// for SwiGLU) products: two tiles halve the workgroups that re-read x, which
-// is what a 64-row call of a wide weight spends most on (TinyLlama's gate|up
-// at 64 rows: 18.4 -> 16.2 us on MI355X; with 2048-2560 columns one tile
-// keeps more workgroups streaming and stays faster).
+// K-split form of the weight stream (the projections of a decode step, the
+// gate|up + SwiGLU launch included): a workgroup owns a BM x WR tile of
+// products over all of K, and its four wavefronts take every fourth 64-wide
+// chunk of K each (128-byte row pieces; the workgroup reads 512 consecutive
+// bytes of a row at a time).  A wavefront keeps its own ring of STAGES chunks
+// of the tile's x and weight rows in LDS, filled by direct-to-LDS loads, and
+// waits only for its own loads: no staging registers and no barrier before
+// the four tiles meet once in LDS.
+//
+// What bounds it is the rate at which a compute unit takes lines it has not
+// in its 32 KB L1: about 53 B/ns, from one chunk in flight per wavefront to
+// six and with the products left out, so the time is 2.2 us plus
+// (BM + WR) rows of K at that rate, per unit.  launch_kstream_tile therefore minimises
+// the rows a compute unit reads.  The weight loads are non-temporal: the weights
+// are read once while x is read again by every workgroup (3-9% over plain
+// loads; non-temporal x loads lose 10-15%).
+// Against four private register-staged quarters of K (us, MI355X, bf16,
+// weights cycled through 2 GB), at 64 / 32 / 4 rows: qkv + norm (2560 x 2048)
+// 8.3 / 7.0 / 5.2 -> 7.3 / 6.1 / 4.4, o (2048 x 2048) 6.5 / 5.0 / 4.7 ->
+// 6.0 / 4.7 / 4.2, gate|up + norm + SwiGLU (11264 x 2048) 16.6 / 14.6 / 11.4 ->
+// 14.3 / 11.4 / 9.9, down (2048 x 5632) 13.1 / 9.5 / 8.3 -> 11.7 / 8.8 / 7.1;
+// within a 64-row step of 22 layers, whose other launches' weights and pages
+// then also stay longer in the memory-side cache, 1489 -> 1436 in all.
 // ---------------------------------------------------------------------------
-// Chunk rows are KC * 2 bytes; pieces are permuted by (piece ^ (row & mask))
-// with mask = min(KC / 8, 16) - 1.
-template <int KC>
-__device__ __forceinline__ int kstream_lds_offset(int row, int piece) {
-  constexpr int kMask = (KC / 8 < 16 ? KC / 8 : 16) - 1;
-  return row * KC + ((piece ^ (row & kMask)) << 3);
-}
-
 // Epilogues of the K-split kernel.
 //   kEpiPlain     y = round(sum)
 //   kEpiNorm      y = round(rsqrt(mean_k(x[r][k]^2) + eps) * sum): the
@@ -350,198 +354,230 @@ __device__ __forceinline__ int kstream_lds_offset(int row, int piece) {
 //   kEpiResidual  y = round(round(sum) + residual[r][n]): the projection
 //                 added to the residual stream, rounded as a separate add is
 enum KstreamEpi : int { kEpiPlain = 0, kEpiNorm = 1, kEpiResidual = 2 };
-template <typename T>
-struct KstreamExtra {
-  float eps = 0.f;
-  const T *residual = nullptr;
-  int64_t residual_stride = 0;
+struct KstreamParams {
+  const void *x;
+  const void *w;
+  void *y;
+  const void *residual;
+  int64_t x_stride;
+  int64_t w_stride;
+  int64_t y_stride;
+  int64_t residual_stride;
+  float eps;
+  int32_t m;
+  int32_t n;           // output columns
+  int32_t k;
+  int32_t tiles_n;
+  int32_t row_blocks;  // of BM rows
 };
 
-// SWIGLU: the workgroup's 16 NT columns j are activation columns; the
-// weight stacks gate rows [0, n) over up rows [n, 2n), each wavefront
-// accumulates both tiles of every column tile over its quarter of K, and
-// the output is round(swiglu_act(round(g), round(u))) (g and u scaled by
-// the row's norm first under kEpiNorm).
-template <typename T, int MT, int KC, bool SWIGLU, int NT, int EPI>
-__global__ void __launch_bounds__(256)
-linear_kstream_kernel(const T *__restrict__ x, int64_t x_stride, const T *__restrict__ w,
-                      int64_t w_stride, T *__restrict__ y, int64_t y_stride, int32_t m,
-                      int32_t n, int32_t k, int32_t k_per_wave, KstreamExtra<T> extra) {
+constexpr int kKsWaves = 4;
+constexpr int kKsChunk = 64;      // k per ring buffer
+constexpr int kKsRowBytes = 128;  // bytes of a chunk row
+constexpr int kKsXcds = 8;
+constexpr int32_t kKsUnits = 256;  // compute units
+
+// 16 bytes per lane from `src` straight to LDS at `lds` + 16 lane (m0 holds the
+// LDS address).  No register is written: vmcnt counts the load, and the LDS
+// bytes are valid after a wait for it.
+template <bool STREAM>
+__device__ __forceinline__ void ks_load_lds(const unsigned char *src, uint32_t lds) {
+  if constexpr (STREAM)
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, off nt"
+        :
+        : "v"(src), "s"(lds)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, off"
+        :
+        : "v"(src), "s"(lds)
+        : "memory");
+}
+
+// Chunks of a ring: what fits 80 KB (two workgroups per compute unit where
+// the grid has that many), at least two.
+constexpr int ks_stages(int rows) {
+  const int fit = 80 * 1024 / (kKsWaves * rows * kKsRowBytes);
+  return fit < 2 ? 2 : (fit > 5 ? 5 : fit);
+}
+
+// SWIGLU: the weight stacks gate rows [0, n) over up rows [n, 2n); a tile's
+// WR weight rows are WR / 2 gate rows and the same up rows, and the output is
+// round(swiglu_act(round(g), round(u))) (g and u scaled by the row's norm
+// first under kEpiNorm).
+template <typename T, int BM, int WR, bool SWIGLU, int EPI>
+__global__ void __launch_bounds__(64 * kKsWaves)
+linear_kstream_kernel(KstreamParams p) {
   using M = SplitMma<T>;
   using vec8 = typename M::vec8;
   static_assert(!(SWIGLU && EPI == kEpiResidual), "the residual epilogue has no SwiGLU form");
-  // blockIdx.y: a block of 16 MT rows of x and y.
-  const int32_t r0 = static_cast<int32_t>(blockIdx.y) * 16 * MT;
-  x += static_cast<int64_t>(r0) * x_stride;
-  y += static_cast<int64_t>(r0) * y_stride;
-  if constexpr (EPI == kEpiResidual) extra.residual += static_cast<int64_t>(r0) * extra.residual_stride;
-  m = min(m - r0, 16 * MT);
-  constexpr int XR = 16 * MT;
-  constexpr int CW = 16 * NT;                  // output columns per workgroup
-  constexpr int WR = SWIGLU ? 2 * CW : CW;     // weight rows per workgroup
-  constexpr int kLanesPerRow = KC / 8;
-  constexpr int kRowsPerLoad = 64 / kLanesPerRow;
-  constexpr int kLoadsX = XR / kRowsPerLoad;
-  constexpr int kLoadsW = WR / kRowsPerLoad;
-  constexpr int kWaveElems = (XR + WR) * KC;
-  constexpr int kItems = MT * 4 * 64;          // floats of one 16-column tile
-  constexpr int kTiles = SWIGLU ? 2 : 1;
-  // The tile sums reuse the staging regions.
-  static_assert(4 * kTiles * NT * kItems * 4 <= 4 * kWaveElems * static_cast<int>(sizeof(T)),
-                "tile sums exceed the staging LDS");
-  extern __shared__ __attribute__((aligned(16))) unsigned char kstream_smem[];
+  constexpr int STAGES = ks_stages(BM + WR);
+  constexpr int MT = BM / 16, NT = WR / 16;
+  constexpr int OC = SWIGLU ? WR / 2 : WR;     // output columns
+  constexpr int kLoads = (BM + WR) / 8;        // load instructions of a chunk: 8 rows each
+  constexpr int kStageBytes = (BM + WR) * kKsRowBytes;
+  constexpr int kSumRow = WR + 4;              // floats; spreads a store's four rows over the banks
+  static_assert(BM % 16 == 0 && WR % 16 == 0 && OC % 8 == 0, "tile");
+  static_assert(kLoads * STAGES <= 63, "vmcnt range");
+  static_assert(BM * kSumRow * 4 <= STAGES * kStageBytes, "tile sums exceed the staging LDS");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char kstream_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  T *xl = reinterpret_cast<T *>(kstream_smem) + wave * kWaveElems;  // [XR][KC]
-  T *wl = xl + XR * KC;                                             // [WR][KC]
   const int l16 = lane & 15;
   const int q4 = lane >> 4;
-  const int32_t n0 = blockIdx.x * CW;
-  const int32_t k0 = min(wave * k_per_wave, k);
-  const int32_t k1 = min(k0 + k_per_wave, k);
-  const int lrow = lane / kLanesPerRow;  // staging: piece lane % (KC/8) of row R i + lane / (KC/8)
-  const int lpiece = lane % kLanesPerRow;
+  // The row blocks of a column tile are consecutive workgroups of one
+  // compute die (id % 8), so its weights come to that die's L2 once.
+  const int32_t group = static_cast<int32_t>(blockIdx.x) / (kKsXcds * p.row_blocks);
+  const int32_t in = static_cast<int32_t>(blockIdx.x) - group * kKsXcds * p.row_blocks;
+  const int32_t tn = group * kKsXcds + in % kKsXcds;
+  if (tn >= p.tiles_n) return;
+  const int32_t m0 = in / kKsXcds * BM;
+  const int32_t n0 = tn * OC;
 
-  const T *xsrc[kLoadsX];
+  // Chunk c of this wavefront is chunk wave + 4 c of K.  K is a multiple of
+  // 32: of a last chunk of 32 the upper four pieces read the lower ones again
+  // and its second k-step is left out.
+  const int32_t all = (p.k + kKsChunk - 1) / kKsChunk;
+  const int32_t chunks = (all - wave + kKsWaves - 1) / kKsWaves;
+  const int32_t half = p.k % kKsChunk != 0 && (all - 1) % kKsWaves == wave ? chunks - 1 : -1;
+
+  // Load i: rows 8 i .. +8 of the chunk, x rows first, the 16-byte piece q of
+  // row r at q ^ (r & 7) so that the lanes of an operand read fall in distinct
+  // banks.  Rows past the matrix read its last row and are not stored.
+  const int lrow = lane >> 3;
+  const int piece = (lane & 7) ^ lrow;
+  const unsigned char *src[kLoads];
 #pragma unroll
-  for (int i = 0; i < kLoadsX; ++i)
-    xsrc[i] = x + static_cast<int64_t>(min(kRowsPerLoad * i + lrow, m - 1)) * x_stride + 8 * lpiece;
-  const T *wsrc[kLoadsW];
-#pragma unroll
-  for (int i = 0; i < kLoadsW; ++i) {
-    const int tr = kRowsPerLoad * i + lrow;  // tile row: gate rows [0, CW), then up rows
-    const int64_t row = SWIGLU ? (tr < CW ? 0 : n) + min(n0 + (tr % CW), n - 1)
-                               : min(n0 + tr, n - 1);
-    wsrc[i] = w + row * w_stride + 8 * lpiece;
+  for (int i = 0; i < kLoads; ++i) {
+    const int64_t at = static_cast<int64_t>(wave) * kKsRowBytes + 16 * piece;
+    if (8 * i < BM) {
+      src[i] = static_cast<const unsigned char *>(p.x) + min(m0 + 8 * i + lrow, p.m - 1) * p.x_stride * 2 + at;
+    } else {
+      const bool up = SWIGLU && 8 * i - BM >= OC;
+      const int64_t row = min(n0 + 8 * i - BM - (up ? OC : 0) + lrow, p.n - 1) + (up ? static_cast<int64_t>(p.n) : 0);
+      src[i] = static_cast<const unsigned char *>(p.w) + row * p.w_stride * 2 + at;
+    }
   }
-
-  vec8 xa[kLoadsX], wa[kLoadsW], xb[kLoadsX], wb[kLoadsW];
-  // Pieces past K read the row's first piece; those past the wavefront's
-  // range but inside K are read and unused.
-  auto load_chunk = [&](int32_t kk, vec8(&xr)[kLoadsX], vec8(&wr)[kLoadsW]) {
-    const int32_t c = kk + 8 * lpiece < k ? kk : -8 * lpiece;
+  unsigned char *ring = kstream_smem + wave * (STAGES * kStageBytes);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char *)ring));
+  const int64_t back = piece >= 4 ? -64 : 0;
+  // Chunks are loaded in order; src moves on with them.
+  auto load = [&](int32_t c, int32_t stage) {
+    const int64_t shift = c == half ? back : 0;
 #pragma unroll
-    for (int i = 0; i < kLoadsX; ++i) xr[i] = *reinterpret_cast<const vec8 *>(xsrc[i] + c);
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i) wr[i] = *reinterpret_cast<const vec8 *>(wsrc[i] + c);
+    for (int i = 0; i < kLoads; ++i) {
+      const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + static_cast<uint32_t>(stage * kStageBytes + i * 1024));
+      if (8 * i < BM)
+        ks_load_lds<false>(src[i] + shift, at);
+      else
+        ks_load_lds<true>(src[i] + shift, at);
+      src[i] += kKsWaves * kKsRowBytes;
+    }
   };
-  f32x4 acc[MT][NT], accu[SWIGLU ? MT : 1][NT];
+
+  f32x4 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) acc[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int mt = 0; mt < (SWIGLU ? MT : 1); ++mt)
-#pragma unroll
-    for (int ct = 0; ct < NT; ++ct) accu[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // The region is private to the wavefront, whose LDS requests are served in
-  // order: compiler barriers order the stores, the operand reads and the
-  // next chunk's stores.
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
   // kEpiNorm: this lane's sums of squares of the x operands it feeds the
   // MFMAs (row 16 mt + l16, eight elements of every k-step in range), taken
   // from the operand registers so they cost no load and overlap the MFMAs.
   float ssq[EPI == kEpiNorm ? MT : 1];
 #pragma unroll
   for (int i = 0; i < (EPI == kEpiNorm ? MT : 1); ++i) ssq[i] = 0.f;
-  auto stage_compute = [&](int32_t kk, const vec8(&xr)[kLoadsX], const vec8(&wr)[kLoadsW]) {
-    __asm__ volatile("" ::: "memory");
+
+  // Chunk c, with FLIGHT chunks loaded after it; LOAD: its buffer then takes
+  // chunk c + STAGES (all operands are in registers before the load is issued).
+  int32_t stage = 0;
+  int32_t c = 0;
+  auto step = [&](auto flight_tag, auto load_tag) {
+    constexpr int FLIGHT = decltype(flight_tag)::value;
+    constexpr bool LOAD = decltype(load_tag)::value;
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads * FLIGHT) : "memory");
+    vec8 a[2][MT], b[2][NT];
+    const unsigned char *at = ring + stage * kStageBytes + l16 * kKsRowBytes;
 #pragma unroll
-    for (int i = 0; i < kLoadsX; ++i)
-      *reinterpret_cast<vec8 *>(xl + kstream_lds_offset<KC>(kRowsPerLoad * i + lrow, lpiece)) = xr[i];
+    for (int s = 0; s < 2; ++s) {
+      const int pc = 16 * ((4 * s + q4) ^ (l16 & 7));
 #pragma unroll
-    for (int i = 0; i < kLoadsW; ++i)
-      *reinterpret_cast<vec8 *>(wl + kstream_lds_offset<KC>(kRowsPerLoad * i + lrow, lpiece)) = wr[i];
-    __asm__ volatile("" ::: "memory");
-    const int32_t steps = min(KC, k1 - kk) >> 5;
+      for (int mt = 0; mt < MT; ++mt) a[s][mt] = *reinterpret_cast<const vec8 *>(at + 16 * mt * kKsRowBytes + pc);
 #pragma unroll
-    for (int st = 0; st < KC / 32; ++st) {
-      if (st >= steps) break;  // uniform
-      const int piece = 4 * st + q4;
-      vec8 b[NT], bu[NT];
+      for (int nt = 0; nt < NT; ++nt) b[s][nt] = *reinterpret_cast<const vec8 *>(at + (BM + 16 * nt) * kKsRowBytes + pc);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    if constexpr (LOAD) load(c + STAGES, stage);
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct) {
-        b[ct] = *reinterpret_cast<const vec8 *>(wl + kstream_lds_offset<KC>(16 * ct + l16, piece));
-        if constexpr (SWIGLU)
-          bu[ct] = *reinterpret_cast<const vec8 *>(wl + kstream_lds_offset<KC>(CW + 16 * ct + l16, piece));
-      }
+    for (int s = 0; s < 2; ++s) {
+      if (s == 1 && c == half) break;  // uniform
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const vec8 a = *reinterpret_cast<const vec8 *>(xl + kstream_lds_offset<KC>(16 * mt + l16, piece));
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-          acc[mt][ct] = M::mma(a, b[ct], acc[mt][ct]);
-          if constexpr (SWIGLU) accu[mt][ct] = M::mma(a, bu[ct], accu[mt][ct]);
-        }
-        if constexpr (EPI == kEpiNorm) ssq[mt] = dot8<T>(a, a, ssq[mt]);
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = M::mma(a[s][mt], b[s][nt], acc[mt][nt]);
+        if constexpr (EPI == kEpiNorm) ssq[mt] = dot8<T>(a[s][mt], a[s][mt], ssq[mt]);
       }
     }
-    __asm__ volatile("" ::: "memory");
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    ++c;
   };
-
-  // Two chunks in flight.  Every iteration issues both register sets'
-  // loads, past the wavefront's last chunk re-reading that chunk (unused),
-  // so the loop head holds the same loads outstanding from the entry and
-  // from the back edge and each set is waited for alone; a load issued on
-  // only some paths would make the wait at the head drain both sets.
-  if (k0 < k1) {
-    const int32_t last = k0 + ((k1 - k0 - 1) / KC) * KC;
-    load_chunk(k0, xa, wa);
-    load_chunk(min(k0 + KC, last), xb, wb);
-    for (int32_t kk = k0; kk < k1; kk += 2 * KC) {
-      stage_compute(kk, xa, wa);
-      load_chunk(min(kk + 2 * KC, last), xa, wa);
-      stage_compute(kk + KC, xb, wb);  // no products past the range
-      load_chunk(min(kk + 3 * KC, last), xb, wb);
-    }
-  }
-
-  // kEpiNorm: a row's sum of squares over its four lanes, then over the
-  // four wavefronts' quarters of K.
-  // Rows of sums [4 waves][XR] past the staging regions.
-  float *ssq_rows = reinterpret_cast<float *>(kstream_smem + 4 * kWaveElems * sizeof(T));
-  if constexpr (EPI == kEpiNorm) {
+  using Yes = std::true_type;
+  using No = std::false_type;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
+  for (int i = 0; i < STAGES; ++i)
+    if (i < chunks) load(i, i);  // uniform
+  while (c + STAGES < chunks) step(std::integral_constant<int, STAGES - 1>{}, Yes{});
+  // At most STAGES chunks are left, all in flight.
+  if constexpr (STAGES >= 5)
+    if (chunks - c >= 5) step(std::integral_constant<int, 4>{}, No{});
+  if constexpr (STAGES >= 4)
+    if (chunks - c >= 4) step(std::integral_constant<int, 3>{}, No{});
+  if constexpr (STAGES >= 3)
+    if (chunks - c >= 3) step(std::integral_constant<int, 2>{}, No{});
+  if (chunks - c >= 2) step(std::integral_constant<int, 1>{}, No{});
+  if (chunks - c >= 1) step(std::integral_constant<int, 0>{}, No{});
+
+  // Sum the four wavefronts' tiles in order: tile row r, weight row j at
+  // sums[wave][r][j].
+  float *sums = reinterpret_cast<float *>(kstream_smem);
+  float *ssq_rows = sums + kKsWaves * BM * kSumRow;  // [4 waves][BM]
+  __syncthreads();  // every wavefront's loads have landed and its operand reads are done
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sums[(wave * BM + 16 * mt + 4 * q4 + r) * kSumRow + 16 * nt + l16] = acc[mt][nt][r];
+    if constexpr (EPI == kEpiNorm) {
       float v = ssq[mt];
       v += __shfl_xor(v, 16, 64);  // the four lanes (l16, q4) of row 16 mt + l16
       v += __shfl_xor(v, 32, 64);
-      if (q4 == 0) ssq_rows[wave * XR + 16 * mt + l16] = v;
+      if (q4 == 0) ssq_rows[wave * BM + 16 * mt + l16] = v;
     }
   }
-  // Sum the four wavefront tiles: item (mt, r, lane) of column tile ct is
-  // y[16 mt + 4 q4 + r][n0 + 16 ct + l16].
-  __syncthreads();  // every wavefront's operand reads are done
-  float *tiles = reinterpret_cast<float *>(kstream_smem);  // [4 waves][kTiles][NT][kItems]
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        tiles[((wave * kTiles) * NT + ct) * kItems + (mt * 4 + r) * 64 + lane] = acc[mt][ct][r];
-        if constexpr (SWIGLU)
-          tiles[((wave * kTiles + 1) * NT + ct) * kItems + (mt * 4 + r) * 64 + lane] = accu[mt][ct][r];
-      }
   __syncthreads();
-  for (int it = threadIdx.x; it < NT * kItems; it += 256) {
-    const int ct = it / kItems;
-    const int item = it - ct * kItems;
+  for (int it = threadIdx.x; it < BM * OC; it += 64 * kKsWaves) {
+    const int r = it / OC;
+    const int j = it - r * OC;
+    const int32_t row = m0 + r;
+    const int32_t col = n0 + j;
+    if (row >= p.m || col >= p.n) continue;
     float sum = 0.f, sumu = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < 4; ++wv) {
-      sum += tiles[((wv * kTiles) * NT + ct) * kItems + item];
-      if constexpr (SWIGLU) sumu += tiles[((wv * kTiles + 1) * NT + ct) * kItems + item];
+    for (int wv = 0; wv < kKsWaves; ++wv) {
+      sum += sums[(wv * BM + r) * kSumRow + j];
+      if constexpr (SWIGLU) sumu += sums[(wv * BM + r) * kSumRow + OC + j];
     }
-    const int mt = item >> 8;
-    const int r = (item >> 6) & 3;
-    const int il = item & 63;
-    const int32_t row = 16 * mt + 4 * (il >> 4) + r;
-    const int32_t col = n0 + 16 * ct + (il & 15);
-    if (row >= m || col >= n) continue;
     if constexpr (EPI == kEpiNorm) {
-      const float sq = ((ssq_rows[row] + ssq_rows[XR + row]) + ssq_rows[2 * XR + row]) +
-                       ssq_rows[3 * XR + row];
-      const float scale = rsqrtf(sq / static_cast<float>(k) + extra.eps);
+      const float sq = ((ssq_rows[r] + ssq_rows[BM + r]) + ssq_rows[2 * BM + r]) + ssq_rows[3 * BM + r];
+      const float scale = rsqrtf(sq / static_cast<float>(p.k) + p.eps);
       sum *= scale;
       sumu *= scale;
     }
@@ -550,286 +586,22 @@ linear_kstream_kernel(const T *__restrict__ x, int64_t x_stride, const T *__rest
       out = from_float<T>(swiglu_act(to_float(from_float<T>(sum)), to_float(from_float<T>(sumu))));
     else if constexpr (EPI == kEpiResidual)
       out = from_float<T>(to_float(from_float<T>(sum)) +
-                          to_float(extra.residual[static_cast<int64_t>(row) * extra.residual_stride + col]));
+                          to_float(static_cast<const T *>(p.residual)[static_cast<int64_t>(row) * p.residual_stride + col]));
     else
       out = from_float<T>(sum);
-    y[static_cast<int64_t>(row) * y_stride + col] = out;
+    static_cast<T *>(p.y)[static_cast<int64_t>(row) * p.y_stride + col] = out;
   }
 }
 
-// Activation-resident form of the K-split kernel (the SwiGLU + RMSNorm
-// launch at 49-64 rows with K = 2048; launch_kstream_mt picks it): each
-// wavefront copies its K quarter of the workgroup's 16 MT rows of x into
-// LDS once, then streams only weights over the column tiles blockIdx.x,
-// blockIdx.x + groups, ... (INFL chunks of 64 k in flight), so a workgroup
-// reads x once instead of once per 64-k chunk of every tile.  Per lane and
-// k-step the MFMA operands, the order of the k-steps, the sums of squares
-// and the epilogue are those of linear_kstream_kernel, so both forms give
-// the same bits.  The outputs of a workgroup's tiles wait in LDS and are
-// stored after the stream (a store inside it would leave the loads' wait
-// counts unknown at the loop head).
-template <typename T, int MT, int NT, bool SWIGLU, int EPI, int INFL, int KQ, int MAXT>
-__global__ void __launch_bounds__(256)
-linear_xres_kernel(const T *__restrict__ x, int64_t x_stride, const T *__restrict__ w,
-                   int64_t w_stride, T *__restrict__ y, int64_t y_stride, int32_t m, int32_t n,
-                   int32_t k, int32_t groups, KstreamExtra<T> extra) {
-  using M = SplitMma<T>;
-  using vec8 = typename M::vec8;
-  constexpr int KC = 64;
-  constexpr int XR = 16 * MT;
-  constexpr int CW = 16 * NT;
-  constexpr int kSteps = KC / 32;
-  constexpr int kItems = MT * 4 * 64;
-  constexpr int kTiles = SWIGLU ? 2 : 1;
-  const int32_t r0 = static_cast<int32_t>(blockIdx.y) * XR;
-  x += static_cast<int64_t>(r0) * x_stride;
-  y += static_cast<int64_t>(r0) * y_stride;
-  if constexpr (EPI == kEpiResidual) extra.residual += static_cast<int64_t>(r0) * extra.residual_stride;
-  m = min(m - r0, XR);
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int l16 = lane & 15;
-  const int q4 = lane >> 4;
-  constexpr int32_t kq = KQ;          // K quarter (the host checks k == 4 KQ)
-  constexpr int32_t xs = kq + 8;      // padded LDS row: rows 16 B apart in the banks
-  constexpr int32_t nch = kq / KC;    // chunks per tile per wavefront
-  static_assert(nch % INFL == 0, "a group of INFL chunks lies in one tile");
-  constexpr int XL = XR * kq / 512;   // x loads per lane
-  const int32_t k0 = wave * kq;
-  const int32_t ntiles = (n + CW - 1) / CW;
-
-  extern __shared__ __attribute__((aligned(16))) unsigned char xres_smem[];
-  // LDS: x quarters [4][XR][xs] | weight staging [4][WR][KC] (its space
-  // holds the tile sums [4][kTiles][NT][kItems] in the epilogue) | row sums
-  // of squares [4][XR] | rounded outputs [MAXT][XR][CW].
-  constexpr int kStageBytes = 4 * (SWIGLU ? 2 * CW : CW) * KC * static_cast<int>(sizeof(T));
-  constexpr int kTileBytes = 4 * kTiles * NT * kItems * 4;
-  constexpr int kRegion = kStageBytes > kTileBytes ? kStageBytes : kTileBytes;
-  T *xq = reinterpret_cast<T *>(xres_smem) + wave * XR * xs;
-  unsigned char *region = xres_smem + 4 * XR * xs * sizeof(T);
-  T *wl = reinterpret_cast<T *>(region) + wave * (SWIGLU ? 2 * CW : CW) * KC;
-  float *tiles = reinterpret_cast<float *>(region);
-  float *ssq_rows = reinterpret_cast<float *>(region + kRegion);
-  T *outs = reinterpret_cast<T *>(ssq_rows + 4 * XR);
-
-  // Weight loads of stream position i (clamped to the last): tile
-  // blockIdx.x + (i / nch) groups, chunk i % nch; lane (l16, q4) of group g,
-  // k-step s holds w[row][kk + 32 s + 8 q4 .. +8].
-  // Weight chunks are loaded as whole 128-byte row pieces (8 lanes per row,
-  // 8 rows per load) and staged in a per-wavefront LDS region before the
-  // MFMA operand reads, as linear_kstream_kernel stages them.  The host
-  // checks nch % INFL == 0, so a group of INFL positions lies in one tile:
-  // load_w(p, s) loads position p + s of such a group (p past the stream
-  // reloads its last group).
-  constexpr int WR = SWIGLU ? 2 * CW : CW;
-  constexpr int kLanesPerRow = KC / 8;
-  constexpr int kRowsPerLoad = 64 / kLanesPerRow;
-  constexpr int kLoadsW = WR / kRowsPerLoad;
-  const int lrow = lane / kLanesPerRow;
-  const int lpiece = lane % kLanesPerRow;
-  // Row pointers of the tile being loaded: tile index lt (clamped to the
-  // last one, whose chunks are reloaded past the stream), chunk lc.
-  const int32_t my_tiles = (ntiles - static_cast<int32_t>(blockIdx.x) + groups - 1) / groups;
-  const T *wsrc[kLoadsW];
-  auto point_w = [&](int32_t lt) {
-    const int32_t n0 = (static_cast<int32_t>(blockIdx.x) + min(lt, my_tiles - 1) * groups) * CW;
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i) {
-      const int tr = kRowsPerLoad * i + lrow;  // tile row: gate rows [0, CW), then up rows
-      const int64_t row = SWIGLU ? (tr < CW ? 0 : n) + min(n0 + (tr % CW), n - 1) : min(n0 + tr, n - 1);
-      wsrc[i] = w + row * w_stride + k0 + 8 * lpiece;
-    }
-  };
-  int32_t lt = 0, lc = 0;
-  point_w(0);
-  // Chunk lc + s of the tile being loaded; past the stream the last tile's
-  // last group again.
-  auto load_w = [&](int s, vec8(&r)[kLoadsW]) {
-    const int32_t c = (lt < my_tiles ? lc : nch - INFL) + s;
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i) r[i] = *reinterpret_cast<const vec8 *>(wsrc[i] + c * KC);
-  };
-  auto next_group = [&]() {
-    lc += INFL;
-    if (lc == nch) {
-      lc = 0;
-      ++lt;
-      point_w(lt);
-    }
-  };
-
-  // x quarter: XR rows x kq (XL loads per lane, lane: 8 consecutive
-  // elements); rows past m read row m - 1.  All of them go out before the
-  // weight prefetch and are written while it is in flight.
-  vec8 wr[INFL][kLoadsW];
-  {
-    vec8 xb[XL];
-#pragma unroll
-    for (int j = 0; j < XL; ++j) {
-      constexpr int kPerRow = kq / 8;  // lanes' pieces per row
-      const int row = (64 * j + lane) / kPerRow;
-      const int col = 8 * ((64 * j + lane) % kPerRow);
-      xb[j] = *reinterpret_cast<const vec8 *>(x + static_cast<int64_t>(min(row, m - 1)) * x_stride + k0 + col);
-    }
-#pragma unroll
-    for (int s = 0; s < INFL; ++s) load_w(s, wr[s]);
-    next_group();
-    __asm__ volatile("" ::: "memory");  // every load above is issued before the first store
-#pragma unroll
-    for (int j = 0; j < XL; ++j) {
-      constexpr int kPerRow = kq / 8;
-      const int row = (64 * j + lane) / kPerRow;
-      const int col = 8 * ((64 * j + lane) % kPerRow);
-      *reinterpret_cast<vec8 *>(xq + row * xs + col) = xb[j];
-    }
-  }
-  __asm__ volatile("" ::: "memory");  // this wavefront's x stores precede its operand reads
-
-  f32x4 acc[MT][NT], accu[SWIGLU ? MT : 1][NT];
-  float ssq[EPI == kEpiNorm ? MT : 1];
-#pragma unroll
-  for (int i = 0; i < (EPI == kEpiNorm ? MT : 1); ++i) ssq[i] = 0.f;
-  auto zero_acc = [&]() {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct) {
-        acc[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (SWIGLU) accu[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-  };
-  zero_acc();
-  auto compute = [&](int32_t c, const vec8(&r)[kLoadsW], bool first) {
-    __asm__ volatile("" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i)
-      *reinterpret_cast<vec8 *>(wl + kstream_lds_offset<KC>(kRowsPerLoad * i + lrow, lpiece)) = r[i];
-    __asm__ volatile("" ::: "memory");
-    const T *xa = xq + l16 * xs + c * KC + 8 * q4;
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const int piece = 4 * s + q4;
-      vec8 b[NT], bu[NT];
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct) {
-        b[ct] = *reinterpret_cast<const vec8 *>(wl + kstream_lds_offset<KC>(16 * ct + l16, piece));
-        if constexpr (SWIGLU)
-          bu[ct] = *reinterpret_cast<const vec8 *>(wl + kstream_lds_offset<KC>(CW + 16 * ct + l16, piece));
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const vec8 a = *reinterpret_cast<const vec8 *>(xa + 16 * mt * xs + 32 * s);
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-          acc[mt][ct] = M::mma(a, b[ct], acc[mt][ct]);
-          if constexpr (SWIGLU) accu[mt][ct] = M::mma(a, bu[ct], accu[mt][ct]);
-        }
-        if constexpr (EPI == kEpiNorm)
-          if (first) ssq[mt] = dot8<T>(a, a, ssq[mt]);
-      }
-    }
-    __asm__ volatile("" ::: "memory");
-  };
-
-  // Every workgroup has a tile (the host keeps groups <= ntiles): no path
-  // skips the stream, so the prefetch above stays ahead of the x stores.
-  int32_t tile = 0, c0 = 0;
-  for (;;) {
-    const bool first = tile == 0;
-#pragma unroll
-    for (int s = 0; s < INFL; ++s) {
-      compute(c0 + s, wr[s], first);
-      load_w(s, wr[s]);
-    }
-    next_group();
-    c0 += INFL;
-    if (c0 < nch) continue;
-    // Tile done: the four wavefront tiles meet in LDS (as linear_kstream_kernel's epilogue).
-    __syncthreads();  // every wavefront's operand reads are done (the sums reuse the staging)
-    if constexpr (EPI == kEpiNorm) {
-      if (first) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          float v = ssq[mt];
-          v += __shfl_xor(v, 16, 64);
-          v += __shfl_xor(v, 32, 64);
-          if (q4 == 0) ssq_rows[wave * XR + 16 * mt + l16] = v;
-        }
-      }
-    }
-#pragma unroll
-    for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          tiles[((wave * kTiles) * NT + ct) * kItems + (mt * 4 + r) * 64 + lane] = acc[mt][ct][r];
-          if constexpr (SWIGLU)
-            tiles[((wave * kTiles + 1) * NT + ct) * kItems + (mt * 4 + r) * 64 + lane] = accu[mt][ct][r];
-        }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NT * kItems / 256; ++j) {
-      const int it = threadIdx.x + 256 * j;
-      const int ct = it / kItems;
-      const int item = it - ct * kItems;
-      float sum = 0.f, sumu = 0.f;
-#pragma unroll
-      for (int wv = 0; wv < 4; ++wv) {
-        sum += tiles[((wv * kTiles) * NT + ct) * kItems + item];
-        if constexpr (SWIGLU) sumu += tiles[((wv * kTiles + 1) * NT + ct) * kItems + item];
-      }
-      const int mt = item >> 8;
-      const int r = (item >> 6) & 3;
-      const int il = item & 63;
-      const int32_t row = 16 * mt + 4 * (il >> 4) + r;
-      if constexpr (EPI == kEpiNorm) {
-        const float sq = ((ssq_rows[row] + ssq_rows[XR + row]) + ssq_rows[2 * XR + row]) +
-                         ssq_rows[3 * XR + row];
-        const float scale = rsqrtf(sq / static_cast<float>(k) + extra.eps);
-        sum *= scale;
-        sumu *= scale;
-      }
-      // Rounded outputs (before the residual add) wait in LDS for the stores
-      // after the stream: [tile][XR][CW].
-      T out;
-      if constexpr (SWIGLU)
-        out = from_float<T>(swiglu_act(to_float(from_float<T>(sum)), to_float(from_float<T>(sumu))));
-      else
-        out = from_float<T>(sum);
-      outs[tile * XR * CW + row * CW + 16 * ct + (il & 15)] = out;
-    }
-    __syncthreads();  // the sums are read before the next tile writes them
-    zero_acc();
-    c0 = 0;
-    if (++tile == my_tiles) break;
-  }
-  // Stores after the stream (a store inside it would leave the loads'
-  // wait counts unknown at the loop head).
-  for (int32_t e = threadIdx.x; e < my_tiles * XR * CW; e += 256) {
-    const int32_t tile = e / (XR * CW);
-    const int32_t rc = e - tile * XR * CW;
-    const int32_t row = rc / CW;
-    const int32_t col = (static_cast<int32_t>(blockIdx.x) + tile * groups) * CW + (rc - row * CW);
-    if (row >= m || col >= n) continue;
-    T out = outs[e];
-    if constexpr (EPI == kEpiResidual)
-      out = from_float<T>(to_float(out) +
-                          to_float(extra.residual[static_cast<int64_t>(row) * extra.residual_stride + col]));
-    y[static_cast<int64_t>(row) * y_stride + col] = out;
-  }
-}
-
-template <typename T, int MT, int KC, bool SWIGLU, int NT, int EPI>
-void launch_kstream(const void *x, int64_t x_stride, const void *w, int64_t w_stride, void *y,
-                    int64_t y_stride, int32_t m, int32_t n, int32_t k, const KstreamExtra<T> &extra,
-                    hipStream_t stream) {
-  const unsigned row_blocks = static_cast<unsigned>((m + 16 * MT - 1) / (16 * MT));
-  const int32_t steps = k / 32;
-  const int32_t k_per_wave = ((steps + 3) / 4) * 32;
-  const size_t lds =
-      static_cast<size_t>(4) * (16 * MT + (SWIGLU ? 32 : 16) * NT) * KC * sizeof(T) +
-      (EPI == kEpiNorm ? static_cast<size_t>(4) * 16 * MT * sizeof(float) : 0);
+template <typename T, int BM, int WR, bool SWIGLU, int EPI>
+void launch_kstream(KstreamParams p, hipStream_t stream) {
+  constexpr int cols = SWIGLU ? WR / 2 : WR;
+  constexpr int staging = kKsWaves * ks_stages(BM + WR) * (BM + WR) * kKsRowBytes;
+  constexpr int sums = kKsWaves * BM * (WR + 4) * 4 + kKsWaves * BM * 4;
+  constexpr int lds = staging > sums ? staging : sums;
+  p.tiles_n = (p.n + cols - 1) / cols;
+  p.row_blocks = (p.m + BM - 1) / BM;
+  auto kernel = &linear_kstream_kernel<T, BM, WR, SWIGLU, EPI>;
   if (lds > 64 * 1024) {
     // Raise the kernel's dynamic LDS limit once per device (a failure shows
     // up as a launch error).
@@ -838,140 +610,49 @@ void launch_kstream(const void *x, int64_t x_stride, const void *w, int64_t w_st
     int device = 0;
     if (hipGetDevice(&device) == hipSuccess && device >= 0 && device < kMaxDevices &&
         !raised[device].load(std::memory_order_acquire)) {
-      if (hipFuncSetAttribute(
-              reinterpret_cast<const void *>(&linear_kstream_kernel<T, MT, KC, SWIGLU, NT, EPI>),
-              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess)
+      if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess)
         raised[device].store(true, std::memory_order_release);
     }
   }
-  hipLaunchKernelGGL((linear_kstream_kernel<T, MT, KC, SWIGLU, NT, EPI>),
-                     dim3((n + 16 * NT - 1) / (16 * NT), row_blocks), dim3(256), lds, stream,
-                     static_cast<const T *>(x), x_stride, static_cast<const T *>(w), w_stride,
-                     static_cast<T *>(y), y_stride, m, n, k, k_per_wave, extra);
+  const unsigned grid = static_cast<unsigned>((p.tiles_n + kKsXcds - 1) / kKsXcds * kKsXcds * p.row_blocks);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kKsWaves), lds, stream, p);
 }
 
-// The activation-resident SwiGLU + RMSNorm launch (linear_xres_kernel):
-// 32-row blocks (MT 2), one 16-column tile per step (NT 1), eight 64-k
-// chunks in flight, 128 column groups per row block (one workgroup per
-// compute unit at 64 rows, each holding at most kXresMaxTiles tiles' outputs
-// in LDS).  Taken for 49-64 rows at K = 2048 (K quarters of 512) when the
-// tiles fit: gate|up + SwiGLU of TinyLlama at 64 rows, 17.3 -> 15.9 us
-// (MI355X, graph-timed, bit-identical); at 17-48 rows it is slower than
-// the K-split form (32 rows 13.5 against 15.7).
-constexpr int kXresMt = 2;
-constexpr int kXresNt = 1;
-constexpr int kXresInflight = 8;
-constexpr int kXresKq = 512;
-constexpr int kXresMaxTiles = 4;
-constexpr int kXresGroups = 128;
-
-size_t xres_lds_bytes(size_t elem) {
-  constexpr int XR = 16 * kXresMt, CW = 16 * kXresNt;
-  const size_t stage = static_cast<size_t>(4) * 2 * CW * 64 * elem;
-  const size_t sums = static_cast<size_t>(4) * 2 * kXresNt * kXresMt * 256 * 4;
-  return static_cast<size_t>(4) * XR * (kXresKq + 8) * elem + (stage > sums ? stage : sums) +
-         static_cast<size_t>(4) * XR * 4 + static_cast<size_t>(kXresMaxTiles) * XR * CW * elem;
-}
-
-bool xres_fits(int32_t m, int32_t n, int32_t k) {
-  const int32_t ntiles = (n + 16 * kXresNt - 1) / (16 * kXresNt);
-  return m > 48 && m <= 64 && k == 4 * kXresKq && ntiles >= kXresGroups &&
-         (ntiles + kXresGroups - 1) / kXresGroups <= kXresMaxTiles;
-}
-
-template <typename T>
-void launch_xres_swiglu_norm(const void *x, int64_t x_stride, const void *w, int64_t w_stride,
-                             void *y, int64_t y_stride, int32_t m, int32_t n, int32_t k,
-                             const KstreamExtra<T> &extra, hipStream_t stream) {
-  auto kernel = &linear_xres_kernel<T, kXresMt, kXresNt, true, kEpiNorm, kXresInflight, kXresKq,
-                                    kXresMaxTiles>;
-  const size_t lds = xres_lds_bytes(sizeof(T));
-  // Raise the kernel's dynamic LDS limit once per device (a failure shows up
-  // as a launch error).
-  constexpr int kMaxDevices = 64;
-  static std::atomic<bool> raised[kMaxDevices];
-  int device = 0;
-  if (hipGetDevice(&device) == hipSuccess && device >= 0 && device < kMaxDevices &&
-      !raised[device].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(lds)) == hipSuccess)
-      raised[device].store(true, std::memory_order_release);
-  }
-  const unsigned row_blocks = static_cast<unsigned>((m + 16 * kXresMt - 1) / (16 * kXresMt));
-  hipLaunchKernelGGL(kernel, dim3(kXresGroups, row_blocks), dim3(256), lds, stream,
-                     static_cast<const T *>(x), x_stride, static_cast<const T *>(w), w_stride,
-                     static_cast<T *>(y), y_stride, m, n, k, kXresGroups, extra);
-}
-
-// Chunk 64 for the SwiGLU form and above 32 rows, else 128.  A workgroup
-// reads 16 (MT + NT) rows of K (x rows and weight rows; twice NT weight
-// rows for SwiGLU), so fewer rows per workgroup means fewer re-reads of x;
-// one workgroup per compute unit is what keeps the split even.  The plain
-// form therefore takes, among workgroups of 1-4 row tiles (MT) and 1-2
-// column tiles (NT) whose grid fits the 256 compute units, the one with the
-// fewest rows (then the larger grid, then one column tile); a grid that
-// fits with none keeps MT = ceil(m / 16), NT = 1.  On MI355X at 64 rows:
-// qkv (2560 columns) MT 2, NT 2 (160 workgroups) 9.2 -> 7.9 us; 2048
-// columns MT 2, NT 1 (256) 8.8 -> 6.5 us; at 33-48 rows qkv MT 1, NT 2
-// (240) 7.5-7.8 -> 6.5-6.6 us.  The SwiGLU form takes MT = ceil(m / 16)
-// and two column tiles from 4096 activation columns.
+// The tile of a call: BM in 16..64 rows and WR in 16..48 weight rows (32..64
+// with SwiGLU, half of them up rows).  A compute unit reads
+// ceil(workgroups / 256) x (BM + WR) rows of K at one rate whatever the tile, so the
+// fewest rows win; among equals the larger grid, then the fewer x rows (o at
+// 64 rows: 16 x 32 6.0 us, 32 x 16 6.2).  Over 4 to 64 rows of TinyLlama's four
+// projections this is within 3% of the best of 24 tiles.  Every tile sums
+// a product in the same order, so the choice changes no bit.
 template <typename T, bool SWIGLU, int EPI>
-void launch_kstream_mt(const void *x, int64_t x_stride, const void *w, int64_t w_stride, void *y,
-                       int64_t y_stride, int32_t m, int32_t n, int32_t k,
-                       const KstreamExtra<T> &extra, hipStream_t stream) {
-  if constexpr (SWIGLU && EPI == kEpiNorm) {
-    if (xres_fits(m, n, k)) {
-      launch_xres_swiglu_norm<T>(x, x_stride, w, w_stride, y, y_stride, m, n, k, extra, stream);
-      return;
-    }
-  }
-  const int32_t row_tiles = (m + 15) / 16;
-  // 64-wide chunks above 32 rows (twice the chunks per wavefront, half the
-  // staging per chunk), 128 up to 32 rows; bit-identical either way (the
-  // k-steps run in the same order).  On MI355X: qkv at 64 rows 9.0 -> 8.2 us,
-  // o 6.7 -> 6.5, down unchanged; at 1..32 rows 64 is 0.5-1.6 us slower.
-  const int kc = SWIGLU || row_tiles > 2 ? 64 : 128;
-  int mt = row_tiles > 4 ? 4 : row_tiles;
-  int nt = 1;
-  if constexpr (SWIGLU) {
-    if (n >= 4096) nt = 2;
-  } else {
-    int best_rows = 1 << 30;
-    int64_t best_grid = 0;
-    for (int cm = 1; cm <= 4 && cm <= row_tiles; ++cm) {
-      for (int cn = 1; cn <= 2; ++cn) {
-        const int64_t grid = static_cast<int64_t>((row_tiles + cm - 1) / cm) *
-                             ((n + 16 * cn - 1) / (16 * cn));
-        if (grid > 256) continue;
-        if (cm + cn < best_rows || (cm + cn == best_rows && grid > best_grid) ||
-            (cm + cn == best_rows && grid == best_grid && cn < nt)) {
-          best_rows = cm + cn;
-          best_grid = grid;
-          mt = cm;
-          nt = cn;
-        }
+void launch_kstream_tile(const KstreamParams &p, hipStream_t stream) {
+  constexpr int kFirst = SWIGLU ? 32 : 16;
+  const int32_t w_rows = SWIGLU ? 2 * p.n : p.n;
+  int bm = 16, wr = kFirst;
+  int64_t best_rows = 0, best_grid = 0;
+  for (int cm = 16; cm <= 64 && cm < p.m + 16; cm += 16)
+    for (int cw = kFirst; cw < kFirst + 48; cw += 16) {
+      const int64_t grid = static_cast<int64_t>((p.m + cm - 1) / cm) * ((w_rows + cw - 1) / cw);
+      const int64_t rows = (grid + kKsUnits - 1) / kKsUnits * (cm + cw);
+      if (best_rows == 0 || rows < best_rows || (rows == best_rows && grid > best_grid)) {
+        best_rows = rows;
+        best_grid = grid;
+        bm = cm;
+        wr = cw;
       }
     }
+#define TF_KSTREAM_CASE(BM)                                                                        \
+  if (bm == BM) {                                                                                  \
+    if (wr == kFirst) return launch_kstream<T, BM, kFirst, SWIGLU, EPI>(p, stream);                \
+    if (wr == kFirst + 16) return launch_kstream<T, BM, kFirst + 16, SWIGLU, EPI>(p, stream);      \
+    return launch_kstream<T, BM, kFirst + 32, SWIGLU, EPI>(p, stream);                             \
   }
-#define TF_KSTREAM_CASE(MT, NT)                                                                \
-  if (mt == MT && nt == NT) {                                                                  \
-    if (kc == 64)                                                                              \
-      launch_kstream<T, MT, 64, SWIGLU, NT, EPI>(x, x_stride, w, w_stride, y, y_stride, m, n, k, \
-                                                 extra, stream);                                  \
-    else if constexpr (!SWIGLU)                                                                \
-      launch_kstream<T, MT, 128, SWIGLU, NT, EPI>(x, x_stride, w, w_stride, y, y_stride, m, n, \
-                                                  k, extra, stream);                              \
-    return;                                                                                    \
-  }
-  TF_KSTREAM_CASE(1, 1)
-  TF_KSTREAM_CASE(2, 1)
-  TF_KSTREAM_CASE(3, 1)
-  TF_KSTREAM_CASE(4, 1)
-  TF_KSTREAM_CASE(1, 2)
-  TF_KSTREAM_CASE(2, 2)
-  TF_KSTREAM_CASE(3, 2)
-  TF_KSTREAM_CASE(4, 2)
+  TF_KSTREAM_CASE(16)
+  TF_KSTREAM_CASE(32)
+  TF_KSTREAM_CASE(48)
+  TF_KSTREAM_CASE(64)
 #undef TF_KSTREAM_CASE
 }
 
@@ -1219,27 +900,32 @@ int32_t kstream_entry(const void *x, int64_t x_row_stride, const void *weight,
   if (align % 16 != 0)
     return fail(TF_ERROR_UNSUPPORTED, "linear_kstream needs 16-byte aligned x and weight rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define TF_KSTREAM_LAUNCH(T)                                                                  \
-  do {                                                                                        \
-    KstreamExtra<T> extra;                                                                    \
-    extra.eps = eps;                                                                          \
-    extra.residual = static_cast<const T *>(residual);                                       \
-    extra.residual_stride = residual_row_stride;                                              \
-    if (swiglu && epi == kEpiNorm)                                                            \
-      launch_kstream_mt<T, true, kEpiNorm>(x, x_row_stride, weight, weight_row_stride, y,     \
-                                           y_row_stride, m, n, k, extra, s);                  \
-    else if (swiglu)                                                                          \
-      launch_kstream_mt<T, true, kEpiPlain>(x, x_row_stride, weight, weight_row_stride, y,    \
-                                            y_row_stride, m, n, k, extra, s);                 \
-    else if (epi == kEpiNorm)                                                                 \
-      launch_kstream_mt<T, false, kEpiNorm>(x, x_row_stride, weight, weight_row_stride, y,    \
-                                            y_row_stride, m, n, k, extra, s);                 \
-    else if (epi == kEpiResidual)                                                             \
-      launch_kstream_mt<T, false, kEpiResidual>(x, x_row_stride, weight, weight_row_stride, y, \
-                                                y_row_stride, m, n, k, extra, s);             \
-    else                                                                                      \
-      launch_kstream_mt<T, false, kEpiPlain>(x, x_row_stride, weight, weight_row_stride, y,   \
-                                             y_row_stride, m, n, k, extra, s);                \
+  KstreamParams p;
+  p.x = x;
+  p.w = weight;
+  p.y = y;
+  p.residual = residual;
+  p.x_stride = x_row_stride;
+  p.w_stride = weight_row_stride;
+  p.y_stride = y_row_stride;
+  p.residual_stride = residual_row_stride;
+  p.eps = eps;
+  p.m = m;
+  p.n = n;
+  p.k = k;
+  p.tiles_n = p.row_blocks = 0;
+#define TF_KSTREAM_LAUNCH(T)                                          \
+  do {                                                                \
+    if (swiglu && epi == kEpiNorm)                                    \
+      launch_kstream_tile<T, true, kEpiNorm>(p, s);                   \
+    else if (swiglu)                                                  \
+      launch_kstream_tile<T, true, kEpiPlain>(p, s);                  \
+    else if (epi == kEpiNorm)                                         \
+      launch_kstream_tile<T, false, kEpiNorm>(p, s);                  \
+    else if (epi == kEpiResidual)                                     \
+      launch_kstream_tile<T, false, kEpiResidual>(p, s);              \
+    else                                                              \
+      launch_kstream_tile<T, false, kEpiPlain>(p, s);                 \
   } while (0)
   if (dtype == TF_DTYPE_BFLOAT16)
     TF_KSTREAM_LAUNCH(__bf16);

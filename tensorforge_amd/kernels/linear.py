@@ -170,10 +170,9 @@ def linear_stream(x: Tensor, weight: Tensor, *, splits: int = 1, output: Tensor 
 
 def linear_kstream(x: Tensor, weight: Tensor, *, output: Tensor | None = None,
                    norm_eps: float | None = None, residual: Tensor | None = None) -> Tensor:
-    """``x [m, k] @ weight[n, k].T`` for m <= 64 with K split over the four
-    wavefronts of workgroups of one or two 16-column tiles, each staging its
-    chunks through LDS with whole-row loads (the form for weights with few
-    64-column tiles).
+    """``x [m, k] @ weight[n, k].T`` for m <= 64 with K split over a
+    workgroup's four wavefronts, each loading its chunks of x and the weight
+    straight to LDS.
 
     ``norm_eps``: the RMSNorm of x's rows applied to the product,
     ``round(rsqrt(mean(x[r]^2) + eps) * (x[r] . weight[n]))``, for a weight
@@ -254,9 +253,9 @@ def linear_swiglu(x: Tensor, gate_up_weight: Tensor, *, output: Tensor | None = 
     ``gate_up_weight`` stacking the gate rows over the up rows (``[2I, k]``)
     -- the stacked projection and its activation in one launch.  The default
     form is bit-identical to :func:`linear_stream` of the stacked weight
-    followed by ``swiglu_gate_up``; ``k_split=True`` splits K over the
-    wavefronts of workgroups of one or two 16-column tiles (bit-identical to
-    :func:`linear_kstream` followed by ``swiglu_gate_up``).  ``norm_eps``
+    followed by ``swiglu_gate_up``; ``k_split=True`` splits K over a
+    workgroup's wavefronts (bit-identical to :func:`linear_kstream` followed
+    by ``swiglu_gate_up``).  ``norm_eps``
     (with ``k_split``): the RMSNorm of x's rows applied to both products
     before the activation, for a weight carrying the norm's gain
     (:func:`fold_norm_gain`).  Returns ``[m, I]`` in ``output`` (allocated
