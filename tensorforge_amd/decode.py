@@ -53,6 +53,7 @@ from torch.nn.attention import SDPBackend, sdpa_kernel
 from tensorforge_amd import _native
 from tensorforge_amd.batch import BatchExecutionResult
 from tensorforge_amd.cache import AppendReservation, PagedKVCache
+from tensorforge_amd.capture import graph_capture
 from tensorforge_amd.kernels import (
     argmax_rows,
     embedding_rms_norm,
@@ -465,7 +466,7 @@ class DecodeGraphBucket:
             torch.cuda.synchronize(self.device)
             warm = time.perf_counter()
             self._graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(self._graph):
+            with graph_capture(self._graph):
                 self._forward()
             if metrics is not None:
                 metrics.capture_count += 1
@@ -933,6 +934,46 @@ class DecodeStepRecord:
     graph: bool = True
 
 
+class _FoldedWeights:
+    """Per layer, the qkv and gate|up weights with the input and
+    post-attention norm gains folded in: made on the first call, shared by
+    every bucket of an executor.  An object of its own, so that buckets refer
+    to the copies and not to their executor: without that cycle an executor's
+    graphs, events and pinned buffers go with its last reference."""
+
+    def __init__(self, weights: DecoderWeights) -> None:
+        self._weights = weights
+        self._copies: list[tuple[Tensor, Tensor]] | None = None
+        self._sources: list[Tensor] = []
+        self._version = 0
+
+    def __call__(self) -> list[tuple[Tensor, Tensor]]:
+        if self._copies is None:
+            layers = self._weights.layers
+            self._copies = [(fold_norm_gain(layer.qkv, layer.input_norm),
+                             fold_norm_gain(layer.gate_up, layer.post_norm)) for layer in layers]
+            self._sources = [tensor for layer in layers
+                             for tensor in (layer.qkv, layer.input_norm, layer.gate_up,
+                                            layer.post_norm)]
+            self._version = sum(t._version for t in self._sources)
+        return self._copies
+
+    def refresh(self) -> bool:
+        """Remake the copies in place if a source was written in place since
+        they were made; whether they were."""
+
+        if self._copies is None:
+            return False
+        version = sum(t._version for t in self._sources)
+        if version == self._version:
+            return False
+        for (qkv, gate_up), layer in zip(self._copies, self._weights.layers):
+            qkv.copy_(fold_norm_gain(layer.qkv, layer.input_norm))
+            gate_up.copy_(fold_norm_gain(layer.gate_up, layer.post_norm))
+        self._version = version
+        return True
+
+
 class BucketedDecodeExecutor:
     """Decode executor over graph buckets (reference:
     BucketedPagedDecodeExecutor, decode_bucket.py:532-666).
@@ -990,9 +1031,6 @@ class BucketedDecodeExecutor:
         self._next_slot = 0
         self._metrics = _MutableMetrics()
         self.step_records: list[DecodeStepRecord] = []
-        self._folded_weights: list[tuple[Tensor, Tensor]] | None = None
-        self._folded_sources: list[Tensor] = []
-        self._folded_version = 0
         # Requests whose logits every pipelined step copies to the host
         # (``watch_logits``), per ring slot: pinned rows and the lanes held.
         self.watch_logits: set[str] = set()
@@ -1000,22 +1038,15 @@ class BucketedDecodeExecutor:
         self._watch_lanes: list[list[tuple[int, str]]] = [[] for _ in range(self._RING)]
         # fuse_norms=False keeps the RMSNorm launches between the
         # projections (the split-K partials path) in every bucket.
-        self._fold = self._folded if fuse_norms else None
+        self._fuse_norms = fuse_norms
+        self._folded: _FoldedWeights | None = None
 
-    def _folded(self) -> list[tuple[Tensor, Tensor]]:
-        """Per layer, the qkv and gate|up weights with the input and
-        post-attention norm gains folded in (made on first use, shared by
-        every bucket of this executor)."""
+    def _fold(self) -> _FoldedWeights | None:
+        """The folded weights that buckets share (None without fused norms)."""
 
-        if self._folded_weights is None:
-            self._folded_weights = [(fold_norm_gain(layer.qkv, layer.input_norm),
-                                     fold_norm_gain(layer.gate_up, layer.post_norm))
-                                    for layer in self.weights.layers]
-            self._folded_sources = [tensor for layer in self.weights.layers
-                                    for tensor in (layer.qkv, layer.input_norm, layer.gate_up,
-                                                   layer.post_norm)]
-            self._folded_version = sum(t._version for t in self._folded_sources)
-        return self._folded_weights
+        if self._fuse_norms and self._folded is None:
+            self._folded = _FoldedWeights(self.weights)
+        return self._folded
 
     def refresh_weights(self) -> bool:
         """Remake the folded qkv and gate|up copies, in place (the captured
@@ -1027,16 +1058,7 @@ class BucketedDecodeExecutor:
         the copies were remade.  Weights replaced by new tensors are not seen
         by graphs captured before; build a new executor for them."""
 
-        if self._folded_weights is None:
-            return False
-        version = sum(t._version for t in self._folded_sources)
-        if version == self._folded_version:
-            return False
-        for (qkv, gate_up), layer in zip(self._folded_weights, self.weights.layers):
-            qkv.copy_(fold_norm_gain(layer.qkv, layer.input_norm))
-            gate_up.copy_(fold_norm_gain(layer.gate_up, layer.post_norm))
-        self._folded_version = version
-        return True
+        return self._folded is not None and self._folded.refresh()
 
     @property
     def vocab_size(self) -> int:
@@ -1091,7 +1113,7 @@ class BucketedDecodeExecutor:
             self._buckets[key] = DecodeGraphBucket(
                 self.weights, self.cache, batch_capacity=batch_capacity,
                 context_capacity=context_capacity, token_state=self.token_state,
-                metrics=self._metrics, folded=self._fold)
+                metrics=self._metrics, folded=self._fold())
         return self._buckets[key]
 
     def _fallback_bucket(self, batch: int, context: int) -> DecodeGraphBucket:
@@ -1106,7 +1128,7 @@ class BucketedDecodeExecutor:
             self._fallbacks[key] = DecodeGraphBucket(
                 self.weights, self.cache, batch_capacity=capacity,
                 context_capacity=config.max_sequence_length, token_state=self.token_state,
-                graph=False, metrics=self._metrics, folded=self._fold)
+                graph=False, metrics=self._metrics, folded=self._fold())
         return self._fallbacks[key]
 
     def capture_all(self) -> None:

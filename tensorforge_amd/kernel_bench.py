@@ -51,6 +51,7 @@ import torch
 
 from tensorforge_amd import workloads
 from tensorforge_amd.cache import PagedKVCache, PagedKVCacheConfig
+from tensorforge_amd.capture import graph_capture
 from tensorforge_amd.decode import (
     BucketedDecodeExecutor,
     DecoderWeights,
@@ -88,7 +89,7 @@ def graph_time_us(run: Callable[[int], None], calls: int, device: torch.device) 
     torch.cuda.current_stream(device).wait_stream(stream)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=stream):
+    with graph_capture(graph, stream=stream):
         for i in range(calls):
             run(i)
     graph.replay()
