@@ -375,8 +375,18 @@ def attention_plan(launch_context: int, batch: int, kv_heads: int, context_capac
     ``element_bytes`` size a token row's slice per kv head.
     """
 
-    fixed = _SPLIT_SIZE is not None
-    split_size = (_SPLIT_SIZE if fixed
+    return _plan(_SPLIT_SIZE, launch_context, batch, kv_heads, context_capacity, attention_path,
+                 slot_limit, head_dim, element_bytes)
+
+
+def _plan(fixed_split: int | None, launch_context: int, batch: int, kv_heads: int,
+          context_capacity: int, attention_path: str, slot_limit: int | None, head_dim: int,
+          element_bytes: int) -> AttentionPlan:
+    """:func:`attention_plan` for a caller-fixed partition size (or None),
+    from its arguments alone."""
+
+    fixed = fixed_split is not None
+    split_size = (fixed_split if fixed
                   else attention_split_size_for(launch_context, batch, kv_heads))
     workgroups = batch * kv_heads
     capacity32 = (context_capacity + 31) // 32 * 32
@@ -411,13 +421,13 @@ def attention_plan(launch_context: int, batch: int, kv_heads: int, context_capac
 def _plan_for(fixed_split: int | None, generic: bool, launch_context: int, batch: int,
               kv_heads: int, context_capacity: int, attention_path: str, slot_limit: int,
               head_dim: int, element_bytes: int) -> tuple[AttentionPlan, int]:
-    """The plan of a call and its launch flags, a function of sizes alone
-    (``fixed_split`` is the caller-fixed partition size :func:`attention_plan`
-    reads); ``generic``: for the generic kernel, which takes fixed partitions
-    and no launch flags beyond them."""
+    """The plan of a call and its launch flags.  Kept for later calls of any
+    thread, so a function of the arguments alone: ``fixed_split`` is the
+    caller-fixed partition size as the call read it; ``generic``: for the generic kernel, which takes fixed
+    partitions and no launch flags beyond them."""
 
-    plan = attention_plan(launch_context, batch, kv_heads, context_capacity, attention_path,
-                          slot_limit, head_dim=head_dim, element_bytes=element_bytes)
+    plan = _plan(fixed_split, launch_context, batch, kv_heads, context_capacity, attention_path,
+                 slot_limit, head_dim, element_bytes)
     if plan.balanced and generic:
         # Fixed partitions sized for about one workgroup per compute unit like
         # any narrow call's (4 rows of 8192 at 32/8 heads, D 128, fp32: 56 us
