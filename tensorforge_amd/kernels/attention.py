@@ -417,13 +417,14 @@ def _plan(fixed_split: int | None, launch_context: int, batch: int, kv_heads: in
     return split if split is not None else one_pass
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)
 def _plan_for(fixed_split: int | None, generic: bool, launch_context: int, batch: int,
               kv_heads: int, context_capacity: int, attention_path: str, slot_limit: int,
               head_dim: int, element_bytes: int) -> tuple[AttentionPlan, int]:
     """The plan of a call and its launch flags.  Kept for later calls of any
-    thread, so a function of the arguments alone: ``fixed_split`` is the
-    caller-fixed partition size as the call read it; ``generic``: for the generic kernel, which takes fixed
+    thread, so a function of the arguments alone (of their types too: 2048.0
+    is no key for 2048): ``fixed_split`` is the caller-fixed partition size as
+    the call read it; ``generic``: for the generic kernel, which takes fixed
     partitions and no launch flags beyond them."""
 
     plan = _plan(fixed_split, launch_context, batch, kv_heads, context_capacity, attention_path,

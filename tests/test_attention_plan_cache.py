@@ -1,6 +1,6 @@
 """The plans that attention calls keep by size (no GPU): a plan filled while
-another thread has fixed a partition size must not
-stay under a key that later calls read."""
+another thread has fixed a partition size, or from arguments of another type,
+must not stay under a key that later calls read."""
 
 from __future__ import annotations
 
@@ -28,3 +28,9 @@ def test_kept_plan_follows_its_key(key, other):
     set_attention_split_size(other)  # as another thread may between the read and the fill
     plan, flags = _plan_for(key, False, *sizes, "auto", 1024, 64, 2)
     assert plan == want and flags == want.flags
+
+
+def test_kept_plan_follows_its_argument_types():
+    first, _ = _plan_for(None, False, 2048.0, 4, 4, 2048, "auto", 1024, 64, 2)
+    plan, _ = _plan_for(None, False, 2048, 4, 4, 2048, "auto", 1024, 64, 2)
+    assert plan is not first and type(plan.split_size) is int and type(plan.num_splits) is int
