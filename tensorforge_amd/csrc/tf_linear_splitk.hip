@@ -377,29 +377,6 @@ constexpr int kKsRowBytes = 128;  // bytes of a chunk row
 constexpr int kKsXcds = 8;
 constexpr int32_t kKsUnits = 256;  // compute units
 
-// 16 bytes per lane from `src` straight to LDS at `lds` + 16 lane (m0 holds the
-// LDS address).  No register is written: vmcnt counts the load, and the LDS
-// bytes are valid after a wait for it.
-template <bool STREAM>
-__device__ __forceinline__ void ks_load_lds(const unsigned char *src, uint32_t lds) {
-  if constexpr (STREAM)
-    asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, off nt"
-        :
-        : "v"(src), "s"(lds)
-        : "memory");
-  else
-    asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, off"
-        :
-        : "v"(src), "s"(lds)
-        : "memory");
-}
-
 // Chunks of a ring: what fits 80 KB (two workgroups per compute unit where
 // the grid has that many), at least two.
 constexpr int ks_stages(int rows) {
@@ -475,9 +452,9 @@ linear_kstream_kernel(KstreamParams p) {
     for (int i = 0; i < kLoads; ++i) {
       const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + static_cast<uint32_t>(stage * kStageBytes + i * 1024));
       if (8 * i < BM)
-        ks_load_lds<false>(src[i] + shift, at);
+        load_lds16(src[i] + shift, at);
       else
-        ks_load_lds<true>(src[i] + shift, at);
+        load_lds16<true>(src[i] + shift, at);
       src[i] += kKsWaves * kKsRowBytes;
     }
   };

@@ -96,20 +96,6 @@ struct PrefillParams {
   float scale_log2;
 };
 
-// 16 bytes per lane from each lane's address straight to LDS at `lds` + 16
-// lane (m0 holds the LDS address; one wait state between its write and the
-// load).  No register is written: vmcnt counts the load, and the LDS bytes
-// are valid after a wait for it.
-__device__ __forceinline__ void prefill_load_lds(const void *src, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(src), "s"(lds)
-      : "memory");
-}
-
 // All but the newest N loads of this wavefront have landed, its LDS reads are
 // done, and so for every wavefront of the workgroup.
 template <int N>
@@ -200,7 +186,7 @@ prefill_attention_kernel(PrefillParams p) {
       if (last < kPrefillChunk - 1) off = offset_of(i, last);  // uniform
       const uint32_t at = lds0 + static_cast<uint32_t>((2 * stage + kv) * kBufBytes) +
                           1024u * static_cast<uint32_t>(wave + kPrefillWaves * (i % (kLoads / 2)));
-      prefill_load_lds(from + off, __builtin_amdgcn_readfirstlane(at));
+      load_lds16(from + off, __builtin_amdgcn_readfirstlane(at));
     }
   };
 #pragma unroll

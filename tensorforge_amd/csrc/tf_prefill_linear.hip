@@ -101,21 +101,6 @@ __device__ __forceinline__ void pl_tile(const PlParams &p, int32_t id, int32_t &
   tm = band * kPlBand + (t - tn * rows);
 }
 
-// 16 bytes per lane from `base` + voffset straight to LDS at `lds` + 16 lane
-// (m0 holds the LDS address; one wait state between its write and the
-// load; the compiler writes m0 itself before any use of its own).  No
-// register is written: vmcnt counts the load, and the LDS bytes are valid
-// after a wait for it.
-__device__ __forceinline__ void pl_load_lds(const void *base, uint32_t voffset, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %0"
-      :
-      : "s"(base), "v"(voffset), "s"(lds)
-      : "memory");
-}
-
 // Every load but the newest `N` of this wavefront has landed and its LDS reads
 // are done; then the workgroup barrier, so that holds for every wavefront.
 template <int N>
@@ -191,8 +176,8 @@ prefill_linear_kernel(PlParams p) {
   // Load i of chunk c into its buffer.
   auto load_one = [&](int32_t c, int32_t stage, int i) {
     const uint32_t at = lds0 + static_cast<uint32_t>(stage * kStageBytes + wave * 1024);
-    pl_load_lds(base[i] + static_cast<int64_t>(c) * kPlRowBytes, voffset[i],
-                __builtin_amdgcn_readfirstlane(at + static_cast<uint32_t>(i * kWaves * 1024)));
+    load_lds16(base[i] + static_cast<int64_t>(c) * kPlRowBytes, voffset[i],
+               __builtin_amdgcn_readfirstlane(at + static_cast<uint32_t>(i * kWaves * 1024)));
   };
 
   f32x4 acc[MT][NT];
