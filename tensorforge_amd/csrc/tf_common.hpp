@@ -80,31 +80,27 @@ __device__ __forceinline__ V load_stream16(const void *p) {
   return __builtin_bit_cast(V, v);
 }
 
-// 16 bytes per lane straight from global memory to LDS at `lds` + 16 lane
-// (m0 takes the LDS address; one wait state between its write and the load).
-// No register is written: vmcnt counts the load, and the LDS bytes are valid
-// after a wait for it.  NT: the nontemporal policy, for data read once.
+// 16 bytes per lane straight from global memory to LDS at `lds` + 16 lane.
+// The LDS address is the instruction's implicit operand m0: bound as one, the
+// compiler writes it and knows what it holds (s_nop: the wait state the load
+// needs after that write).  No register is written: vmcnt counts the load, and
+// the LDS bytes are valid after a wait for it.  NT: the nontemporal policy,
+// for data read once.
 template <bool NT = false>
 __device__ __forceinline__ void load_lds16(const void *src, uint32_t lds) {
   if constexpr (NT)
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                 :
-                 : "v"(src), "s"(lds)
-                 : "memory", "m0");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(src), "{m0}"(lds) : "memory");
   else
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(src), "s"(lds)
-                 : "memory", "m0");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds) : "memory");
 }
 
 // The same from `base` + each lane's offset.  `base` must come from scalar
 // instructions: one that a vector instruction wrote needs five wait states.
 __device__ __forceinline__ void load_lds16(const void *base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0"
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %0"
                :
-               : "s"(base), "v"(offset), "s"(lds)
-               : "memory", "m0");
+               : "s"(base), "v"(offset), "{m0}"(lds)
+               : "memory");
 }
 
 // ---------------------------------------------------------------------------
