@@ -360,14 +360,17 @@ prefill_attention_kernel(PrefillParams p) {
 }
 
 template <typename T, int D, int QH>
-void launch_prefill(const PrefillParams &p, int32_t ntiles, hipStream_t stream) {
-  const unsigned grid = static_cast<unsigned>(ntiles) * static_cast<unsigned>(p.kv_heads * (p.group / QH));
-  hipLaunchKernelGGL((prefill_attention_kernel<T, D, QH>), dim3(grid), dim3(64 * kPrefillWaves), 0,
-                     stream, p);
+int32_t launch_prefill(const PrefillParams &p, int32_t ntiles, hipStream_t stream) {
+  // A launch counts its threads in 32 bits.
+  const int64_t grid = static_cast<int64_t>(ntiles) * p.kv_heads * (p.group / QH);
+  if (grid * (64 * kPrefillWaves) > 0xffffffffll) return fail(TF_ERROR_UNSUPPORTED, "grid too large");
+  hipLaunchKernelGGL((prefill_attention_kernel<T, D, QH>), dim3(static_cast<unsigned>(grid)),
+                     dim3(64 * kPrefillWaves), 0, stream, p);
+  return check_launch("prefill_attention");
 }
 
 template <typename T, int D>
-void launch_prefill_qh(const PrefillParams &p, int32_t ntiles, int32_t heads_per_wave,
+int32_t launch_prefill_qh(const PrefillParams &p, int32_t ntiles, int32_t heads_per_wave,
                        hipStream_t stream) {
   // Query heads per wavefront (a power of two dividing the group): as asked,
   // else one at head_dim 32 and wherever two would leave fewer than
@@ -384,22 +387,20 @@ void launch_prefill_qh(const PrefillParams &p, int32_t ntiles, int32_t heads_per
   if (qh > kMax) qh = kMax;
   if (qh > p.group) qh = p.group;
   switch (qh) {
-    case 1: launch_prefill<T, D, 1>(p, ntiles, stream); break;
-    case 2: launch_prefill<T, D, 2>(p, ntiles, stream); break;
-    case 4: launch_prefill<T, D, 4>(p, ntiles, stream); break;
-    default:
-      if constexpr (kMax >= 8) launch_prefill<T, D, 8>(p, ntiles, stream);
-      break;
+    case 1: return launch_prefill<T, D, 1>(p, ntiles, stream);
+    case 2: return launch_prefill<T, D, 2>(p, ntiles, stream);
+    case 4: return launch_prefill<T, D, 4>(p, ntiles, stream);
+    default: return launch_prefill<T, D, kMax>(p, ntiles, stream);
   }
 }
 
 template <typename T>
-void launch_prefill_dim(const PrefillParams &p, int32_t head_dim, int32_t ntiles,
-                        int32_t heads_per_wave, hipStream_t stream) {
+int32_t launch_prefill_dim(const PrefillParams &p, int32_t head_dim, int32_t ntiles,
+                           int32_t heads_per_wave, hipStream_t stream) {
   switch (head_dim) {
-    case 32: launch_prefill_qh<T, 32>(p, ntiles, heads_per_wave, stream); break;
-    case 64: launch_prefill_qh<T, 64>(p, ntiles, heads_per_wave, stream); break;
-    default: launch_prefill_qh<T, 128>(p, ntiles, heads_per_wave, stream); break;
+    case 32: return launch_prefill_qh<T, 32>(p, ntiles, heads_per_wave, stream);
+    case 64: return launch_prefill_qh<T, 64>(p, ntiles, heads_per_wave, stream);
+    default: return launch_prefill_qh<T, 128>(p, ntiles, heads_per_wave, stream);
   }
 }
 
@@ -461,8 +462,6 @@ extern "C" int32_t tf_prefill_attention(const void *q, int64_t q_row_stride, con
   p.scale_log2 = scale * kPrefillLog2e;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == TF_DTYPE_BFLOAT16)
-    launch_prefill_dim<__bf16>(p, head_dim, num_tiles, heads_per_wave, s);
-  else
-    launch_prefill_dim<_Float16>(p, head_dim, num_tiles, heads_per_wave, s);
-  return check_launch("prefill_attention");
+    return launch_prefill_dim<__bf16>(p, head_dim, num_tiles, heads_per_wave, s);
+  return launch_prefill_dim<_Float16>(p, head_dim, num_tiles, heads_per_wave, s);
 }
