@@ -8,6 +8,7 @@ import pytest
 from tensorforge_amd import _native
 
 FAKE = 0x1000
+UNSUPPORTED = 2  # TF_ERROR_UNSUPPORTED
 
 
 @pytest.mark.parametrize(("tiles", "query_heads", "kv_heads", "head_dim", "heads_per_wave"), [
@@ -23,5 +24,5 @@ def test_a_grid_past_the_launch_limit_is_refused(tiles, query_heads, kv_heads, h
     status = launch.tf_prefill_attention(
         FAKE, width, FAKE, kv_heads * head_dim, FAKE, kv_heads * head_dim, FAKE, width, FAKE, tiles,
         query_heads, kv_heads, head_dim, 1.0, heads_per_wave, _native.TF_DTYPE_BFLOAT16, None)
-    assert status == _native.TF_ERROR_UNSUPPORTED
+    assert status == UNSUPPORTED
     assert b"grid too large" in _native.library().tf_last_error()
