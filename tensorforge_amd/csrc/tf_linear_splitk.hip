@@ -5,8 +5,9 @@
 //     with both operands staged through LDS by whole-row loads;
 //   * tf_linear_swiglu -- its form for the stacked gate|up weight with the
 //     SwiGLU in the epilogue;
-//   * tf_linear_kstream / tf_linear_kswiglu -- K split over the wavefronts
-//     of 16-column workgroups, for narrow weights and for gate|up + SwiGLU.
+//   * tf_linear_kstream / tf_linear_kswiglu -- K split over a workgroup's
+//     wavefronts, each on its own ring of direct-to-LDS loads, for the
+//     projections of a decode step.
 //
 // Split-K form:
 //   partials[s][m][n] = sum over k in slice s of x[m][k] * w[n][k]   (fp32)
@@ -322,27 +323,25 @@ linear_stream_kernel(const T *__restrict__ x, int64_t x_stride, const T *__restr
 // ---------------------------------------------------------------------------
 // K-split form of the weight stream (the projections of a decode step, the
 // gate|up + SwiGLU launch included): a workgroup owns a BM x WR tile of
-// products over all of K, and its four wavefronts take every fourth 64-wide
-// chunk of K each (128-byte row pieces; the workgroup reads 512 consecutive
-// bytes of a row at a time).  A wavefront keeps its own ring of STAGES chunks
-// of the tile's x and weight rows in LDS, filled by direct-to-LDS loads, and
-// waits only for its own loads: no staging registers and no barrier before
-// the four tiles meet once in LDS.
+// products over all of K, and its four wavefronts take a quarter of K each.
+// A wavefront keeps its own ring of STAGES 64-wide chunks (128-byte row
+// pieces) of the tile's x and weight rows in LDS, filled by direct-to-LDS
+// loads, and waits only for its own loads: no staging registers and no
+// barrier before the four tiles meet once in LDS.
 //
 // What bounds it is the rate at which a compute unit takes lines it has not
 // in its 32 KB L1: about 53 B/ns, from one chunk in flight per wavefront to
-// six and with the products left out, so the time is 2.2 us plus
-// (BM + WR) rows of K at that rate, per unit.  launch_kstream_tile therefore minimises
-// the rows a compute unit reads.  The weight loads are non-temporal: the weights
-// are read once while x is read again by every workgroup (3-9% over plain
-// loads; non-temporal x loads lose 10-15%).
-// Against four private register-staged quarters of K (us, MI355X, bf16,
-// weights cycled through 2 GB), at 64 / 32 / 4 rows: qkv + norm (2560 x 2048)
-// 8.3 / 7.0 / 5.2 -> 7.3 / 6.1 / 4.4, o (2048 x 2048) 6.5 / 5.0 / 4.7 ->
-// 6.0 / 4.7 / 4.2, gate|up + norm + SwiGLU (11264 x 2048) 16.6 / 14.6 / 11.4 ->
-// 14.3 / 11.4 / 9.9, down (2048 x 5632) 13.1 / 9.5 / 8.3 -> 11.7 / 8.8 / 7.1;
-// within a 64-row step of 22 layers, whose other launches' weights and pages
-// then also stay longer in the memory-side cache, 1489 -> 1436 in all.
+// nine and with the products left out, so the time of a weight of a few MB is
+// 2.2 us plus (BM + WR) rows of K at that rate, per unit (qkv and o at 64
+// rows: 7.1 and 5.9 us).  Larger ones add the memory's time: gate|up's 46 MB
+// are 8.6 us at the copy rate.
+// Against register-staged chunks of the same quarters (us, MI355X, bf16,
+// weights cycled through 2 GB) at 64 / 33 / 17 / 4 rows:
+//   qkv + norm (2560 x 2048)              8.1 / 6.9 / 6.8 / 5.6 -> 7.5 / 6.2 / 6.1 / 4.8
+//   o + residual (2048 x 2048)            6.5 / 6.2 / 4.9 / 4.8 -> 6.0 / 5.7 / 4.4 / 4.3
+//   gate|up + norm + SwiGLU (11264 x 2048) 15.8 / 14.6 / 12.5 / 11.4 -> 13.9 / 11.6 / 10.3 / 9.4
+//   down + residual (2048 x 5632)         12.7 / 11.9 / 8.4 / 8.3 -> 12.0 / 9.9 / 7.7 / 7.3
+//   4096 x 14336 + residual               38.5 / 33.0 / 25.7 / 21.9 -> 37.2 / 30.8 / 23.7 / 19.4
 // ---------------------------------------------------------------------------
 // Epilogues of the K-split kernel.
 //   kEpiPlain     y = round(sum)
@@ -369,6 +368,7 @@ struct KstreamParams {
   int32_t k;
   int32_t tiles_n;
   int32_t row_blocks;  // of BM rows
+  int32_t stream;      // weights by nontemporal loads
 };
 
 constexpr int kKsWaves = 4;
@@ -417,12 +417,14 @@ linear_kstream_kernel(KstreamParams p) {
   const int32_t m0 = in / kKsXcds * BM;
   const int32_t n0 = tn * OC;
 
-  // Chunk c of this wavefront is chunk wave + 4 c of K.  K is a multiple of
-  // 32: of a last chunk of 32 the upper four pieces read the lower ones again
-  // and its second k-step is left out.
-  const int32_t all = (p.k + kKsChunk - 1) / kKsChunk;
-  const int32_t chunks = (all - wave + kKsWaves - 1) / kKsWaves;
-  const int32_t half = p.k % kKsChunk != 0 && (all - 1) % kKsWaves == wave ? chunks - 1 : -1;
+  // This wavefront's quarter of K, in whole k-steps of 32.  Of a last chunk of
+  // 32 the upper four pieces read the lower ones again and its second k-step
+  // is left out.
+  const int32_t k_per_wave = (p.k / 32 + kKsWaves - 1) / kKsWaves * 32;
+  const int32_t k0 = min(wave * k_per_wave, p.k);
+  const int32_t k1 = min(k0 + k_per_wave, p.k);
+  const int32_t chunks = (k1 - k0 + kKsChunk - 1) / kKsChunk;
+  const int32_t half = (k1 - k0) % kKsChunk != 0 ? chunks - 1 : -1;
 
   // Load i: rows 8 i .. +8 of the chunk, x rows first, the 16-byte piece q of
   // row r at q ^ (r & 7) so that the lanes of an operand read fall in distinct
@@ -432,7 +434,7 @@ linear_kstream_kernel(KstreamParams p) {
   const unsigned char *src[kLoads];
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) {
-    const int64_t at = static_cast<int64_t>(wave) * kKsRowBytes + 16 * piece;
+    const int64_t at = static_cast<int64_t>(k0) * 2 + 16 * piece;
     if (8 * i < BM) {
       src[i] = static_cast<const unsigned char *>(p.x) + min(m0 + 8 * i + lrow, p.m - 1) * p.x_stride * 2 + at;
     } else {
@@ -448,15 +450,21 @@ linear_kstream_kernel(KstreamParams p) {
   // Chunks are loaded in order; src moves on with them.
   auto load = [&](int32_t c, int32_t stage) {
     const int64_t shift = c == half ? back : 0;
+    auto each = [&](auto stream_tag) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + static_cast<uint32_t>(stage * kStageBytes + i * 1024));
-      if (8 * i < BM)
-        load_lds16(src[i] + shift, at);
-      else
-        load_lds16<true>(src[i] + shift, at);
-      src[i] += kKsWaves * kKsRowBytes;
-    }
+      for (int i = 0; i < kLoads; ++i) {
+        const uint32_t at = __builtin_amdgcn_readfirstlane(lds0 + static_cast<uint32_t>(stage * kStageBytes + i * 1024));
+        if (8 * i < BM)
+          load_lds16(src[i] + shift, at);
+        else
+          load_lds16<decltype(stream_tag)::value>(src[i] + shift, at);
+        src[i] += kKsRowBytes;
+      }
+    };
+    if (p.stream)  // uniform
+      each(std::true_type{});
+    else
+      each(std::false_type{});
   };
 
   f32x4 acc[MT][NT];
@@ -597,29 +605,51 @@ void launch_kstream(KstreamParams p, hipStream_t stream) {
 }
 
 // The tile of a call: BM in 16..64 rows and WR in 16..48 weight rows (32..64
-// with SwiGLU, half of them up rows).  A compute unit reads
-// ceil(workgroups / 256) x (BM + WR) rows of K at one rate whatever the tile, so the
-// fewest rows win; among equals the larger grid, then the fewer x rows (o at
-// 64 rows: 16 x 32 6.0 us, 32 x 16 6.2).  Over 4 to 64 rows of TinyLlama's four
-// projections this is within 3% of the best of 24 tiles.  Every tile sums
-// a product in the same order, so the choice changes no bit.
+// with SwiGLU, half of them up rows), and whether its weights stream past the
+// caches.  A compute unit reads ceil(workgroups / 256) x (BM + WR) rows of K
+// at 53 B/ns whatever the tile, so the fewest rows win; then, since each row
+// block reads the weights and blocks of long rows do not keep together in L2,
+// the fewest blocks above kKsShortK (4096 x 4096 at 17 rows: one block 8.3 us,
+// two 12.0), then the larger grid (qkv at 64 rows: 216 workgroups in four
+// blocks 7.4 us, 160 in two 7.8).
+// Nontemporal weights (TinyLlama's qkv at 4 rows 5.3 -> 4.7 us, gate|up 10.7
+// -> 9.5) need whole lines per row piece (rows of 1984 bytes: 3.7 -> 4.3) and
+// weights that would not stay in the caches anyway (1536 x 1536 at 33 rows
+// 4.7 -> 5.1), and they come from memory again for a row block that falls out
+// of step with the others: long rows and a last block of few rows, which runs
+// ahead (2048 x 5632 at 17 rows 7.9 -> 8.9 us, at 33 rows 10.0 -> 12.3; in
+// full blocks, 32 and 64 rows, 9.6 -> 9.2 and 12.5 -> 12.2).
+// Over 1 to 64 rows of 39 weights of 0.1 to 268 MB the choice is 1.3% slower
+// than the best of 24 forms.  Every form sums a product in the same order, so
+// the choice changes no bit.
+constexpr int64_t kKsCached = 6000000;  // bytes of weights up to which loads stay temporal
+constexpr int32_t kKsShortK = 2048;     // K up to which row blocks keep together
+
 template <typename T, bool SWIGLU, int EPI>
-void launch_kstream_tile(const KstreamParams &p, hipStream_t stream) {
+void launch_kstream_tile(KstreamParams p, hipStream_t stream) {
   constexpr int kFirst = SWIGLU ? 32 : 16;
-  const int32_t w_rows = SWIGLU ? 2 * p.n : p.n;
+  const int64_t w_rows = SWIGLU ? 2 * static_cast<int64_t>(p.n) : p.n;
+  // Each further row block: a tenth of the weights' time at 8 TB/s.
+  const float block_us = p.k <= kKsShortK ? 0.f : 0.1f * static_cast<float>(w_rows * p.k) * 2.f / 8e6f;
   int bm = 16, wr = kFirst;
-  int64_t best_rows = 0, best_grid = 0;
+  float best = 0.f;
+  int64_t best_grid = 0;
   for (int cm = 16; cm <= 64 && cm < p.m + 16; cm += 16)
     for (int cw = kFirst; cw < kFirst + 48; cw += 16) {
-      const int64_t grid = static_cast<int64_t>((p.m + cm - 1) / cm) * ((w_rows + cw - 1) / cw);
+      const int64_t blocks = (p.m + cm - 1) / cm;
+      const int64_t grid = blocks * ((w_rows + cw - 1) / cw);
       const int64_t rows = (grid + kKsUnits - 1) / kKsUnits * (cm + cw);
-      if (best_rows == 0 || rows < best_rows || (rows == best_rows && grid > best_grid)) {
-        best_rows = rows;
+      const float cost = static_cast<float>(rows * p.k) * 2.f / 53e3f + block_us * static_cast<float>(blocks - 1);
+      if (best_grid == 0 || cost < best || (cost == best && grid > best_grid)) {
+        best = cost;
         best_grid = grid;
         bm = cm;
         wr = cw;
       }
     }
+  const uintptr_t lines = reinterpret_cast<uintptr_t>(p.w) | static_cast<uintptr_t>(p.w_stride * 2);
+  p.stream = lines % kKsRowBytes == 0 && w_rows * p.k * 2 >= kKsCached &&
+             (p.m <= bm || p.k <= kKsShortK || p.m % bm == 0);
 #define TF_KSTREAM_CASE(BM)                                                                        \
   if (bm == BM) {                                                                                  \
     if (wr == kFirst) return launch_kstream<T, BM, kFirst, SWIGLU, EPI>(p, stream);                \
@@ -890,7 +920,7 @@ int32_t kstream_entry(const void *x, int64_t x_row_stride, const void *weight,
   p.m = m;
   p.n = n;
   p.k = k;
-  p.tiles_n = p.row_blocks = 0;
+  p.tiles_n = p.row_blocks = p.stream = 0;
 #define TF_KSTREAM_LAUNCH(T)                                          \
   do {                                                                \
     if (swiglu && epi == kEpiNorm)                                    \
