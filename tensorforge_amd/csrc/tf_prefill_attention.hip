@@ -304,6 +304,9 @@ prefill_attention_kernel(PrefillParams p) {
     }
 #pragma unroll
     for (int h = 0; h < J / 2; ++h) {
+      // A step of 32 keys past the tile's own is left out: all its weights
+      // are 0, but 0 times a value that is not finite is not.
+      if (h > 0 && t0 + k0 + 32 * h >= kend) break;  // wavefront-uniform
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
         const unsigned char *rd = vb + v_at[n] + (k0 + 32 * h) * kRowBytes;
