@@ -351,7 +351,9 @@ prefill_attention_kernel(PrefillParams p) {
     float l = l_run[hq];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    // A query sees a key, so l is 0 only where every score is -inf: then 0 / 0,
+    // the NaN of a softmax over nothing.
+    const float inv = 1.f / l;
     T *dst = orow + static_cast<int64_t>(h0 + hq) * D;
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
