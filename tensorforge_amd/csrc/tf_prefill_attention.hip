@@ -55,7 +55,8 @@ constexpr int kPrefillChunk = 64;  // key tokens per LDS buffer
 constexpr float kPrefillFloor = -3e38f;  // running maximum before the first key
 constexpr float kPrefillMost = 256.f;    // weight that makes the maximum rise
 constexpr int kPrefillXcds = 8;
-constexpr int64_t kPrefillPairs = 600;   // workgroups from which a wavefront serves two heads
+// Workgroups from which a wavefront serves two heads.
+constexpr int64_t prefill_pairs(int head_dim) { return head_dim >= 128 ? 500 : (head_dim >= 64 ? 600 : 1200); }
 
 template <typename T>
 struct PrefillMfma;
@@ -96,11 +97,10 @@ struct PrefillParams {
   float scale_log2;
 };
 
-// All but the newest N loads of this wavefront have landed, its LDS reads are
-// done, and so for every wavefront of the workgroup.
-template <int N>
+// This wavefront's loads have landed, its LDS reads are done, and so for every
+// wavefront of the workgroup.
 __device__ __forceinline__ void prefill_wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
 }
 
 template <typename T, int D, int QH>
@@ -118,9 +118,8 @@ prefill_attention_kernel(PrefillParams p) {
   constexpr int kRowsPer256 = D >= 128 ? 1 : 128 / D;
   constexpr int kRowBytes = 2 * D;
   constexpr int kBufBytes = kPrefillChunk * kRowBytes;  // K or V of a chunk
-  constexpr int kStages = D <= 64 ? 3 : 2;
   constexpr int kSub = D <= 64 ? 64 : 32;  // keys whose operands are held at once
-  __shared__ __attribute__((aligned(1024))) unsigned char ring[kStages][2][kBufBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[2][2][kBufBytes];
   auto swizzle = [](int row) { return (row / kRowsPer256) & (kPieces - 1); };
 
   const int tid = threadIdx.x;
@@ -189,9 +188,7 @@ prefill_attention_kernel(PrefillParams p) {
       load_lds16(from + off, __builtin_amdgcn_readfirstlane(at));
     }
   };
-#pragma unroll
-  for (int c = 0; c < kStages - 1; ++c)
-    if (c < nch) load_chunk(c, c);
+  load_chunk(0, 0);
 
   vec8 qf[QH][KS];  // B operand: q[token i0 + l16][head h0 + hq][32 ks + 8 q4 .. +8]
   {
@@ -225,9 +222,10 @@ prefill_attention_kernel(PrefillParams p) {
     for (int n = 0; n < NB; ++n) acc[hq][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // Keys [t0 + k0, t0 + k0 + kSub) of the chunk at t0.
-  auto compute = [&](int32_t t0, const unsigned char *kb, const unsigned char *vb, int k0) {
-    constexpr int J = kSub / 16;
+  // Keys [t0 + k0, t0 + k0 + KEYS) of the chunk at t0.
+  auto compute = [&](int32_t t0, const unsigned char *kb, const unsigned char *vb, int k0, auto keys_tag) {
+    constexpr int KEYS = decltype(keys_tag)::value;
+    constexpr int J = KEYS / 16;
     vec8 kf[J][KS];
 #pragma unroll
     for (int j = 0; j < J; ++j)
@@ -236,7 +234,7 @@ prefill_attention_kernel(PrefillParams p) {
         kf[j][ks] = *reinterpret_cast<const vec8 *>(kb + k_at[ks] + (k0 + 16 * j) * kRowBytes);
     // Causal mask: needed when some key of the step lies past the tile's
     // first query token (a query's own token bounds its keys in the prompt).
-    const bool masked = t0 + k0 + kSub - 1 > i0;
+    const bool masked = t0 + k0 + KEYS - 1 > i0;
     const int32_t limit = qt - t0 - k0 - 4 * q4;  // key 16 j + r (of q4 = 0) is seen up to this
     vec8 pf[QH][J / 2];
     // Every head's scores and weights before any of the rare paths below, so
@@ -268,14 +266,18 @@ prefill_attention_kernel(PrefillParams p) {
       for (int i = 0; i < 4 * J; ++i)
         pr[hq][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[hq][i], p.scale_log2, -m_run[hq]));
     };
-    float top = 0.f;
+    bool raise = t0 + k0 == s;  // uniform; the first keys raise the maxima in any case
+    if (!raise) {
+      float top = 0.f;
 #pragma unroll
-    for (int hq = 0; hq < QH; ++hq) {
-      weights(hq);
+      for (int hq = 0; hq < QH; ++hq) {
+        weights(hq);
 #pragma unroll
-      for (int i = 0; i < 4 * J; i += 2) top = fmaxf(fmaxf(pr[hq][i], pr[hq][i + 1]), top);
+        for (int i = 0; i < 4 * J; i += 2) top = fmaxf(fmaxf(pr[hq][i], pr[hq][i + 1]), top);
+      }
+      raise = __ballot(top > kPrefillMost) != 0;
     }
-    if (__ballot(top > kPrefillMost) != 0) {  // uniform: raise the maxima
+    if (raise) {
 #pragma unroll
       for (int hq = 0; hq < QH; ++hq) {
         float mx = sc[hq][0] * p.scale_log2;
@@ -319,27 +321,32 @@ prefill_attention_kernel(PrefillParams p) {
     }
   };
 
-  // Chunk c waits for its own loads (the next chunk's may stay in flight);
-  // past the barrier every wavefront is done with chunk c - 1, whose buffer
-  // takes chunk c + kStages - 1.
-  int32_t stage = 0;
+  // Chunk c waits for its loads; past the barrier every wavefront is done with
+  // chunk c - 1, whose buffer takes chunk c + 1.
+  using Keys32 = std::integral_constant<int, 32>;
+  using Keys64 = std::integral_constant<int, 64>;
   for (int32_t c = 0; c < nch; ++c) {
-    if (kStages > 2 && c + 1 < nch)
-      prefill_wait_barrier<(kStages - 2) * kLoads>();
-    else
-      prefill_wait_barrier<0>();
-    if (c + kStages - 1 < nch) load_chunk(c + kStages - 1, stage == 0 ? kStages - 1 : stage - 1);
-    if (c < my_nch) {  // wavefront-uniform
-      const unsigned char *kb = ring[stage][0];
-      const unsigned char *vb = ring[stage][1];
-#pragma unroll
-      for (int k0 = 0; k0 < kPrefillChunk; k0 += kSub) {
-        // The second half of a chunk past the tile's keys has nothing to add.
-        if (k0 > 0 && s + kPrefillChunk * c + k0 >= kend) break;
-        compute(s + kPrefillChunk * c, kb, vb, k0);
-      }
+    prefill_wait_barrier();
+    if (c + 1 < nch) load_chunk(c + 1, (c + 1) & 1);
+    if (c >= my_nch) continue;  // wavefront-uniform, as all below
+    const unsigned char *kb = ring[c & 1][0];
+    const unsigned char *vb = ring[c & 1][1];
+    const int32_t t0 = s + kPrefillChunk * c;
+    const bool whole = kend - t0 > 32;  // the second half has keys of the tile
+    if constexpr (kSub == 32) {
+      compute(t0, kb, vb, 0, Keys32{});
+      if (whole) compute(t0, kb, vb, 32, Keys32{});
+    } else if constexpr (QH > 1) {
+      compute(t0, kb, vb, 0, Keys64{});
+    } else {
+      // A form for half a chunk: a third of a short prompt's work.  With
+      // several heads its registers cost more (8,058 tokens at 32/4 heads, D
+      // 64: 57 -> 64 us).
+      if (whole)
+        compute(t0, kb, vb, 0, Keys64{});
+      else
+        compute(t0, kb, vb, 0, Keys32{});
     }
-    stage = stage + 1 == kStages ? 0 : stage + 1;
   }
 
   // Lane-partial sums -> per-column sums; write the query tokens of the prompt.
@@ -378,17 +385,17 @@ template <typename T, int D>
 int32_t launch_prefill_qh(const PrefillParams &p, int32_t ntiles, int32_t heads_per_wave,
                        hipStream_t stream) {
   // Query heads per wavefront (a power of two dividing the group): as asked,
-  // else one at head_dim 32 and wherever two would leave fewer than
-  // kPrefillPairs workgroups -- a call then waits for its longest chain of
-  // chunks, which one head shortens -- and two otherwise, which read each
-  // chunk's operands half as often (MI355X, us with one / two heads: 271
-  // tokens 5.8 / 7.4, 2048 30.4 / 34.4, 3 x 1000 25.9 / 24.3, 19 prompts of
-  // 8,058 tokens 71.6 / 57.4 at 32/4 heads, D 64; 2048 53.7 / 52.2, 4096 +
-  // 2051 + 777 249 / 185 at 32/8, D 128; 19.6 / 24.9 at 8/2, D 32).  At most
-  // 4 at head_dim 128, for registers.
+  // else one where two would leave fewer than prefill_pairs workgroups -- a
+  // call then waits for its longest chain of chunks, which one head shortens
+  // -- and two otherwise, which read each chunk's operands half as often.
+  // MI355X, us with one / two heads: D 64 at 16/1 heads 4096 tokens (512
+  // pairs) 61.9 / 65.6, 19 prompts of 8,058 tokens at 32/4 (2176) 61.3 / 52.8;
+  // D 128 at 32/8 1000 tokens (256) 22.1 / 26.0, at 16/2 8 x 500 (512) 21.2 /
+  // 19.7; D 32 at 8/2 the 8,058 tokens (544) 20.6 / 25.4, 128 x 130 tokens
+  // (1536) 16.3 / 11.0.  At most 4 at head_dim 128, for registers.
   constexpr int kMax = D >= 128 ? 4 : 8;
   const int64_t pairs = static_cast<int64_t>(ntiles) * p.kv_heads * ((p.group + 1) / 2);
-  int32_t qh = heads_per_wave > 0 ? heads_per_wave : (D >= 64 && pairs >= kPrefillPairs ? 2 : 1);
+  int32_t qh = heads_per_wave > 0 ? heads_per_wave : (pairs >= prefill_pairs(D) ? 2 : 1);
   if (qh > kMax) qh = kMax;
   if (qh > p.group) qh = p.group;
   switch (qh) {
