@@ -144,16 +144,18 @@ rms_norm_kernel(const T *__restrict__ inputs, const T *__restrict__ residual,
   V *y = reinterpret_cast<V *>(output + row * columns);
   const V *w = reinterpret_cast<const V *>(weight);
 
-  // Long rows take their vectors in groups of kAhead, so that the gains in
-  // flight do not push the row's cache out of the registers.
-  constexpr int kAhead = VECS < 2 ? 1 : 2;
-  constexpr bool kGainAhead = AHEAD && VECS <= kAhead;
+  // Vectors whose loads are issued together; alone (1) a vector is loaded only
+  // by the lanes that have one, which costs a branch and saves the loads.
+  constexpr int kMost = VEC == 1 || VECS < 4 ? 2 : VECS;
+  constexpr int kAhead = PARTIALS || (RESIDUAL && !AHEAD) || VECS < 2 ? 1 : (AHEAD ? kMost : 2);
+  constexpr bool kGainAhead = AHEAD && VECS <= 2 && VECS <= kAhead;
   float cache[VECS][VEC];
   V wv[kAhead];
   float sq = 0.f;
 #pragma unroll
   for (int k0 = 0; k0 < VECS; k0 += kAhead) {
     if (VECS > kAhead && k0 * static_cast<int32_t>(blockDim.x) >= nvec) break;
+    if (VECS > 1 && kAhead == 1 && static_cast<int32_t>(threadIdx.x + k0 * blockDim.x) >= nvec) continue;
     V xv[kAhead], rv[kAhead];
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) {
@@ -279,20 +281,22 @@ void launch_norm(const void *inputs, const void *residual, const void *weight,
     else
       run(&rms_norm_kernel<T, VEC, VECS, AHEAD, RESIDUAL, false>, nullptr, 0, GatherRows{});
   };
-  // A kernel for one, two, or up to the register cache's vectors per lane;
-  // gains ahead while every row's workgroup is resident at once (256 compute
-  // units of about eight), past which the call is bound by HBM.
-  constexpr std::true_type kYes{};
-  constexpr std::false_type kNo{};
-  constexpr std::integral_constant<int, 1> kOne{};
-  constexpr std::integral_constant<int, 2> kTwo{};
-  const bool ahead = rows <= 2048;
-  if (nvec > 2 * threads)
-    launch(std::integral_constant<int, max_vecs<VEC>()>{}, kNo);
-  else if (nvec > threads)
-    ahead ? launch(kTwo, kYes) : launch(kTwo, kNo);
+  // A kernel for one, two, four, or up to the register cache's vectors per
+  // lane.  Loads run ahead where the call waits for them: while every row's
+  // workgroup is resident at once (256 compute units of about eight), and for
+  // the residual norm, which streams three arrays, while they fit the L1s (32
+  // KB each): 1024 x 4096 bf16 6.8 us ahead, 6.4 not; 1024 x 2048 4.7 and 4.8.
+  const bool ahead = RESIDUAL && !partials ? rows * columns * static_cast<int64_t>(sizeof(T)) < (8 << 20)
+                                           : rows <= 2048;
+  auto launch_vecs = [&](auto vecs) { ahead ? launch(vecs, std::true_type{}) : launch(vecs, std::false_type{}); };
+  if (nvec <= threads)
+    launch_vecs(std::integral_constant<int, 1>{});
+  else if (nvec <= 2 * threads)
+    launch_vecs(std::integral_constant<int, 2>{});
+  else if (nvec <= 4 * threads)
+    launch_vecs(std::integral_constant<int, 4>{});
   else
-    ahead ? launch(kOne, kYes) : launch(kOne, kNo);
+    launch_vecs(std::integral_constant<int, max_vecs<VEC>()>{});
 }
 
 template <typename T, bool RESIDUAL>
