@@ -751,12 +751,17 @@ def _prefill_packed(weights: DecoderWeights, cache: PagedKVCache, prompts: dict[
     positions = longs[1]
     eps = config.rms_norm_eps
     dtype = weights.embedding.dtype
-    residual = torch.empty((total, config.hidden_size), dtype=dtype, device=device)
-    # The prompts' ids come from the host rows (source -1); the lane state is
-    # not read.
-    residual, h = embedding_rms_norm(longs[0], longs[2], longs[0], weights.embedding,
-                                     weights.layers[0].input_norm, eps, x_output=residual,
-                                     norm_output=torch.empty_like(residual))
+    input_norm = weights.layers[0].input_norm
+    if weights.embedding.is_contiguous():
+        residual = torch.empty((total, config.hidden_size), dtype=dtype, device=device)
+        # The prompts' ids come from the host rows (source -1); the lane state
+        # is not read.
+        residual, h = embedding_rms_norm(longs[0], longs[2], longs[0], weights.embedding,
+                                         input_norm, eps, x_output=residual,
+                                         norm_output=torch.empty_like(residual))
+    else:  # a table of padded rows, say
+        residual = F.embedding(longs[0], weights.embedding)
+        h = rms_norm(residual, input_norm, eps)
     native = None
     if _NativePrefill.supported(weights, cache, total):
         native = _NativePrefill(weights, cache, total, positions, ints, tiles)
