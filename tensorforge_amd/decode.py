@@ -731,7 +731,8 @@ class _NativePrefill:
 def _dense(tensor: Tensor, shape: tuple[int, ...], cache: PagedKVCache) -> bool:
     return (tensor.shape == shape and tensor.dtype == cache.config.dtype
             and tensor.device == cache.config.device and tensor.is_contiguous()
-            and tensor.data_ptr() % 16 == 0)
+            and tensor.data_ptr() % 16 == 0
+            and not (tensor.requires_grad and torch.is_grad_enabled()))
 
 
 def _prefill_packed(weights: DecoderWeights, cache: PagedKVCache, prompts: dict[str, list[int]],

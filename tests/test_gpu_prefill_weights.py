@@ -1,4 +1,5 @@
-"""Which weights a prefill takes: an embedding table with padded rows too."""
+"""Which weights a prefill takes: an embedding table with padded rows, and none
+that gradients are to reach (the kernels are inference-only)."""
 
 from __future__ import annotations
 
@@ -41,3 +42,16 @@ def test_prefill_takes_an_embedding_of_padded_rows(device):
     got = _prefill(dataclasses.replace(weights, embedding=padded), cache)
     assert not want.errors and not got.errors
     assert all(torch.equal(got.logits[request_id], want.logits[request_id]) for request_id in PROMPTS)
+
+
+@pytest.mark.parametrize("name", ["o_proj", "down"])
+def test_prefill_refuses_weights_that_require_grad(device, name):
+    weights, cache = _model(device)
+    want = _prefill(weights, cache)
+    getattr(weights.layers[1], name).requires_grad_(True)
+    result = _prefill(weights, cache)
+    assert not result.logits and all("inference-only" in message for message in result.errors.values())
+    with torch.no_grad():
+        result = _prefill(weights, cache)
+    assert not result.errors
+    assert all(torch.equal(result.logits[request_id], want.logits[request_id]) for request_id in PROMPTS)
