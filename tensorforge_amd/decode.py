@@ -611,9 +611,13 @@ def _validate_prompt(weights: DecoderWeights, cache: PagedKVCache, request_id: s
 
 # Prefills of at most this many tokens run their projections on the library's
 # own prefill GEMM, one native call per layer; longer ones keep hipBLASLt for
-# all but the gate|up projection (MI355X, TinyLlama: at 2000 rows qkv / o /
-# down 27.6 / 22.1 / 54.6 us against 27.2 / 20.9 / 46.3, at 8058 rows 85 / 52 /
-# 133 against 74 / 61 / 157; gate|up with its SwiGLU 433 against 346).
+# all but the gate|up projection.  MI355X, TinyLlama, us own / hipBLASLt at 2304,
+# 4096 and 8058 rows: qkv 29.9 / 27.4, 54.3 / 43.0 and 71.7 / 82.9 (behind from
+# 1500 to 6000 rows, ahead only at the last), o 28.1 / 27.5, 35.8 / 33.9 and
+# 60.5 / 50.1, down 69.9 / 56.1, 77.8 / 76.2 and 139 / 122; gate|up with its
+# SwiGLU 110 / 106, 182 / 195 and 329 / 405.  Up to 2048 tokens the layer call's
+# host time and launches outweigh that: prefills of 1 to 2048 tokens at eight
+# geometries (hidden 1024 to 5120) take 0.27 to 1.06 of the time without it.
 PREFILL_NATIVE_TOKENS = 2048
 
 
