@@ -31,10 +31,11 @@
 // computed again.  Softmax in base 2, fp32 accumulation, one rounding of the
 // output.
 //
-// MI355X: 19 prompts of 8,058 tokens at 32/4 heads, D 64 92.9 -> 57.4 us (613
-// TFLOP/s of causal attention), 4096 + 2051 + 777 tokens at 32/8, D 128 310
-// -> 185 us (958), one prompt of 271 9.2 -> 5.8 us, against 32-key chunks
-// staged through registers with the maximum looked for in every chunk.
+// MI355X: 19 prompts of 8,058 tokens at 32/4 heads, D 64 92.5 -> 52.5 us (673
+// TFLOP/s of causal attention), 4096 + 2051 + 777 tokens at 32/8, D 128 311
+// -> 193 us (917), one prompt of 271 9.9 -> 6.0 us, 64 prompts of 20 7.3 -> 7.6,
+// against 32-key chunks staged through registers with the maximum looked for in
+// every chunk.
 //
 // Reference semantics: the causal scaled-dot-product attention of prefill,
 // tensorforge/runtime/prefill.py:84-88 (causal mask over the padded

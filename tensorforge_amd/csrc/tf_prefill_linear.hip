@@ -329,8 +329,9 @@ int32_t launch_prefill_linear(PlParams p, hipStream_t stream) {
 // 1.2x).  Against the library GEMM (plus the SwiGLU launch for gate|up):
 // 271 rows qkv 11.9 -> 8.8 us, o 11.4 -> 8.3, gate|up 33.0 -> 26.7, down
 // 27.7 -> 16.3; 1500 rows 21.8 -> 21.2, 19.3 -> 17.4, 84.7 -> 67.3,
-// 46.4 -> 43.4; 8058 rows gate|up 433 -> 346 (o 52.2 -> 60.7 and down
-// 133 -> 157: above 2048 rows the callers keep the library for those).
+// 46.4 -> 43.4; 8058 rows gate|up 405 -> 329 (o 50.1 -> 60.5, down 122 -> 139,
+// and qkv at 4096 rows 43.0 -> 54.3, at 6000 47.9 -> 58.1: above 2048 rows the
+// callers keep the library for those three).
 // A workgroup is bound by the latency of its loads in flight (up to 147 KB)
 // at few rows, and by the products at many: at 8058 rows the 256 x 256 tile
 // runs at 1.18 PFLOP/s, 1.6 with every row aliased to one (the clock under

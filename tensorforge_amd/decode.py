@@ -191,7 +191,7 @@ def _project(x: Tensor, weight: Tensor, output: Tensor | None = None) -> Tensor:
     LDS-staged weight stream (linear_stream: 24.6-25.0 us against 30.4-30.7
     for hipBLASLt at 32000 x 2048; 12.6-12.8 us against 12.5-14.7 at
     11264 x 2048).  Narrower weights with K >= 1024 (the stacked q/k/v)
-    take the K-split weight stream (linear_kstream: 4.4-7.4 us at 1..64 rows
+    take the K-split weight stream (linear_kstream: 4.3-7.1 us at 1..64 rows
     against 5.7-12.9 for linear_rows and 11.2-11.9 for hipBLASLt at
     2560 x 2048).  Other weights up to 16 rows use the K-split MFMA kernel
     (linear_rows) when small (<= 8M elements), where the library GEMM
@@ -339,8 +339,8 @@ class DecodeGraphBucket:
                 self.partials_down = torch.empty((self.split_down, b, config.hidden_size),
                                                  dtype=torch.float32, device=device)
         # The MLP's gate|up projection with SwiGLU in its epilogue, K split
-        # over a workgroup's wavefronts (TinyLlama 11264 x 2048: 10.3-11.5 us
-        # at 1..32 rows and 14.3 at 64, against 14.7-16.8 and 18.8 for the
+        # over a workgroup's wavefronts (TinyLlama 11264 x 2048: 9.2-10.6 us
+        # at 1..32 rows and 13.2 at 64, against 14.7-16.8 and 18.8 for the
         # best projection + SwiGLU pair).
         probe_h = torch.empty((b, config.hidden_size), dtype=dtype, device=device)
         self.fused_gate_up = linear_rows_supported(probe_h, layer0.gate_up)
